@@ -95,8 +95,9 @@ int sepia_gpu_matvec_q(int ggml_type, SepiaGpuBuf *w, size_t w_off, SepiaGpuBuf 
  * bit-identical to the reference's dequantize_row (also F16). */
 int sepia_gpu_dequant_rows(int ggml_type, SepiaGpuBuf *raw, size_t raw_off, SepiaGpuBuf *out, int64_t n);
 
-/* src/sepia_gpu.h:209 and :226 -- banded attention is outside this
- * library's scope (the quantized-weight path); both log and return 0. */
+/* src/sepia_gpu.h:209 and :226 -- the relative-position projection, and
+ * banded GQA attention with an online softmax (head dims that are a multiple
+ * of 4 up to 128, up to 16 query heads per kv head). */
 int sepia_gpu_rel_project(SepiaGpuBuf *r_vec, SepiaGpuBuf *rel_proj, SepiaGpuBuf *rel_logits,
                           int64_t T, int64_t H, int64_t d_rel, int64_t rel_extent);
 int sepia_gpu_banded_attn(SepiaGpuBuf *q, SepiaGpuBuf *k, SepiaGpuBuf *v, SepiaGpuBuf *rel_logits,

@@ -63,8 +63,8 @@ enum {
     K_PF_ROUTE_M,
     /* u32 fill (counter words of caller-provided scratch) */
     K_FILL_U32,
-    /* attention (kernels/attn.h): relative-position projection, banded attention partials and fold */
-    K_REL_PROJECT, K_ATTN_PARTIAL, K_ATTN_COMBINE,
+    /* attention (kernels/attn.h): relative-position projection, banded attention and the fold of its splits */
+    K_REL_PROJECT, K_ATTN_BOUNDS, K_ATTN_WAVE, K_ATTN_WAVE_D, K_ATTN_TILE, K_ATTN_TILE_D, K_ATTN_COMBINE,
     /* prefill projections of Q2_K / Q3_K / Q4_K on the int8 matrix cores (kernels/prefill_q.h) */
     K_PF_QUANT, K_PF_GATEUP_Q, K_PF_DOWN_Q,
     /* prefill projections of the real checkpoint's formats on the f16 matrix cores (kernels/prefill_h.h) */
@@ -95,7 +95,8 @@ static const char *const k_names[K_COUNT] = {
     "sepia_mq_gateup", "sepia_mq_down",
     "sepia_pf_route", "sepia_pf_select", "sepia_pf_group", "sepia_pf_gateup", "sepia_pf_down", "sepia_pf_combine",
     "sepia_pf_split", "sepia_pf_route_m", "sepia_fill_u32",
-    "sepia_rel_project_f32", "sepia_attn_partial", "sepia_attn_combine",
+    "sepia_rel_project_f32", "sepia_attn_bounds", "sepia_attn_wave", "sepia_attn_wave_d",
+    "sepia_attn_tile", "sepia_attn_tile_d", "sepia_attn_combine",
     "sepia_pf_quant", "sepia_pf_gateup_q", "sepia_pf_down_q",
     "sepia_ph_quant", "sepia_ph_gateup", "sepia_ph_down",
     "sepia_read_probe", "sepia_read_probe_dma",
@@ -136,6 +137,7 @@ static const TypeInfo k_types[] = {
 #define TILE_TMAX 3
 #define TILE_MAX_COLS (2 * 16 * TILE_NT)
 #define TILE_CUS 256    /* MI355X compute units: the grid aims at one workgroup per CU */
+#define MQ_CUS 256      /* the same, for the matrix-core kernels */
 typedef struct {
     int32_t U, S, T, tiles;
 } TileGeo;
@@ -1239,17 +1241,116 @@ int sepia_gpu_rel_project_off(SepiaGpuBuf *r_vec, SepiaGpuBuf *rel_proj, size_t 
 }
 
 /* Banded attention (reference src/sepia_gpu.h:226; CPU semantics
- * src/sepia.c:1211-1247): per token a launch of span workgroups per kv head
- * writes per-head partials to scratch, a second launch folds them. Tokens go
- * ATT_TB a launch pair, their kv bounds and tau in the kernel arguments (the
- * caller's host arrays are read here and need not outlive the call). Mirrors
- * struct AttnTok in kernels/attn.h. */
+ * src/sepia.c:1211-1247; kernels/attn.h): a launch of tile or wave
+ * workgroups per kv head, split over the kv range where the tiles alone
+ * leave the chip idle, and a fold of the splits. The caller's bounds and tau
+ * go in the kernel arguments, or for more than ATT_TB tokens first to scratch
+ * (either way the host arrays are read here and need not outlive the call).
+ * The structs mirror those of kernels/attn.h. */
 #define ATT_TB 64
-#define ATT_CH 128
+#define ATT_BB 256
+#define ATT_KC 32           /* kv rows per step of sepia_attn_tile */
+#define ATT_WAVE_STEP 64    /* and per round of a sepia_attn_wave workgroup */
+#define ATT_FOLD 1024       /* splits sepia_attn_combine folds at most */
+#define ATT_TMAX 32768      /* tokens per launch */
+#define ATT_WAVE_ROWS 32    /* rows (tokens x heads of a kv head) up to which the wave kernel runs */
 typedef struct {
     int32_t lo[ATT_TB], hi[ATT_TB];
     float tau[ATT_TB];
 } AttnTok;
+typedef struct {
+    int32_t lo[ATT_BB], hi[ATT_BB];
+    float tau[ATT_BB];
+} AttnTokB;
+typedef struct {
+    const float *q, *k, *v, *rel;
+    const int32_t *gtok;
+    float *out;
+    double *part;
+    int64_t q_pos_base, kv_dim;
+    int32_t T, H, Hkv, Dh, R, nsplit, span, TT;
+    float inv_head_dim;
+} AttnArgs;
+
+/* Bytes of scratch a call may use: what there is while the stream is being
+ * captured, else any amount. */
+static size_t scratch_limit(void) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(g_stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone) return SIZE_MAX;
+    return g_scratch ? g_scratch_len - CNT_BYTES : 0;
+}
+
+/* Tokens t0 .. t0 + T - 1 (T <= ATT_TMAX) of a call whose arguments are checked. */
+static int attn_launch(const char *op, AttnArgs a, int64_t t0, const int64_t *kv_lo, const int64_t *kv_hi,
+                       const float *tau) {
+    const int64_t T = a.T, G = a.H / a.Hkv;
+    /* Few rows: the waves of a workgroup split the kv range of 16 rows and
+     * read k and v once each from global memory. Many: 64 rows share the k
+     * and v rows through LDS. */
+    const int wave = T * G <= ATT_WAVE_ROWS;
+    const int64_t step = wave ? ATT_WAVE_STEP : ATT_KC;
+    a.TT = (int32_t)((wave ? 16 : 64) / G);
+    const int64_t tiles = (T + a.TT - 1) / a.TT;
+    int64_t n_max = 0;   /* the longest kv range of a tile */
+    for (int64_t b = 0; b < T; b += a.TT) {
+        int64_t lo = INT64_MAX, hi = -1;
+        for (int64_t t = b; t < T && t < b + a.TT; t++) {
+            if (kv_lo[t0 + t] < lo) lo = kv_lo[t0 + t];
+            if (kv_hi[t0 + t] > hi) hi = kv_hi[t0 + t];
+        }
+        if (hi - lo + 1 > n_max) n_max = hi - lo + 1;
+    }
+    /* splits: two workgroups a CU (what their registers and LDS allow), each
+     * of whole steps; fewer where a capture holds the scratch to what there is */
+    const int64_t steps = (n_max + step - 1) / step;
+    int64_t nsplit = (2 * MQ_CUS + a.Hkv * tiles - 1) / (a.Hkv * tiles);
+    if (2 * a.Hkv * tiles > 2 * MQ_CUS) nsplit = 1;
+    if (nsplit > steps) nsplit = steps;
+    if (nsplit > ATT_FOLD) nsplit = ATT_FOLD;
+    const size_t bounds = T > ATT_TB ? ((size_t)T * 12 + 255) & ~(size_t)255 : 0;
+    const size_t per = (size_t)T * (size_t)a.H * (size_t)(a.Dh + 2) * 8, limit = scratch_limit();
+    while (nsplit > 1 && bounds + (size_t)nsplit * per > limit) nsplit--;
+    const int64_t span = (steps + nsplit - 1) / nsplit * step;
+    nsplit = (n_max + span - 1) / span;
+    a.nsplit = (int32_t)nsplit;
+    a.span = span > 0x7FFFFFFF ? 0x7FFFFFFF : (int32_t)span;
+    a.gtok = NULL;
+    a.part = NULL;
+    if (bounds || nsplit > 1) {
+        uint8_t *s = (uint8_t *)scratch(bounds + (nsplit > 1 ? (size_t)nsplit * per : 0), op);
+        if (!s) return 0;
+        if (bounds) a.gtok = (const int32_t *)s;
+        if (nsplit > 1) a.part = (double *)(s + bounds);
+    }
+    AttnTok tok;
+    memset(&tok, 0, sizeof tok);
+    if (!bounds) {
+        for (int64_t i = 0; i < T; i++) {
+            tok.lo[i] = (int32_t)kv_lo[t0 + i];
+            tok.hi[i] = (int32_t)kv_hi[t0 + i];
+            tok.tau[i] = tau[t0 + i];
+        }
+    }
+    for (int64_t b = 0; bounds && b < T; b += ATT_BB) {
+        AttnTokB tb;
+        int32_t n = (int32_t)(T - b < ATT_BB ? T - b : ATT_BB), b32 = (int32_t)b, T32 = (int32_t)T;
+        memset(&tb, 0, sizeof tb);
+        for (int32_t i = 0; i < n; i++) {
+            tb.lo[i] = (int32_t)kv_lo[t0 + b + i];
+            tb.hi[i] = (int32_t)kv_hi[t0 + b + i];
+            tb.tau[i] = tau[t0 + b + i];
+        }
+        void *a_b[] = { &tb, &n, &b32, &T32, &a.gtok };
+        if (!launch(K_ATTN_BOUNDS, 1, ATT_BB, a_b, op)) return 0;
+    }
+    void *a_p[] = { &a, &tok };
+    const int kern = a.Dh == 128 ? (wave ? K_ATTN_WAVE : K_ATTN_TILE) : (wave ? K_ATTN_WAVE_D : K_ATTN_TILE_D);
+    if (!launch3(kern, (unsigned)a.Hkv, (unsigned)tiles, (unsigned)nsplit, 256, 0, a_p, op))
+        return 0;
+    if (nsplit == 1) return 1;
+    void *a_c[] = { &a.part, &a.H, &a.Dh, &a.nsplit, &a.out };
+    return launch2(K_ATTN_COMBINE, (unsigned)a.H, (unsigned)T, 128, 0, a_c, op);
+}
 
 int sepia_gpu_banded_attn(SepiaGpuBuf *q, SepiaGpuBuf *k, SepiaGpuBuf *v, SepiaGpuBuf *rel_logits,
                           SepiaGpuBuf *attn_out, const int64_t *kv_lo, const int64_t *kv_hi, const float *tau,
@@ -1266,7 +1367,7 @@ int sepia_gpu_banded_attn(SepiaGpuBuf *q, SepiaGpuBuf *k, SepiaGpuBuf *v, SepiaG
         LOG("%s: head dim %lld not supported (a multiple of 4 up to 128)", op, (long long)Dh);
         return 0;
     }
-    int64_t max_hi = 0, max_n = 0;
+    int64_t max_hi = 0;
     for (int64_t t = 0; t < T; t++) {
         if (kv_lo[t] < 0 || kv_hi[t] < kv_lo[t] || kv_hi[t] > q_pos_base + t || kv_hi[t] > 0x7FFFFFFF) {
             LOG("%s: token %lld: kv range [%lld, %lld] outside [0, q_pos %lld]", op, (long long)t,
@@ -1274,7 +1375,6 @@ int sepia_gpu_banded_attn(SepiaGpuBuf *q, SepiaGpuBuf *k, SepiaGpuBuf *v, SepiaG
             return 0;
         }
         if (kv_hi[t] > max_hi) max_hi = kv_hi[t];
-        if (kv_hi[t] - kv_lo[t] + 1 > max_n) max_n = kv_hi[t] - kv_lo[t] + 1;
     }
     if (kv_dim % 4) {
         LOG("%s: kv_dim %lld is not a multiple of 4 (k and v rows are read 16 bytes at a time)", op,
@@ -1287,44 +1387,27 @@ int sepia_gpu_banded_attn(SepiaGpuBuf *q, SepiaGpuBuf *k, SepiaGpuBuf *v, SepiaG
     if (!chk(q, 0, qb, op, "q") || !chk(k, 0, kvb, op, "k") || !chk(v, 0, kvb, op, "v") ||
         !chk(rel_logits, 0, rlb, op, "rel_logits") || !chk(attn_out, 0, qb, op, "attn_out"))
         return 0;
-    /* spans: enough workgroups to cover the CUs, each span whole steps */
-    const int64_t tb = T < ATT_TB ? T : ATT_TB;
-    int64_t nsplit = (1024 + Hkv * tb - 1) / (Hkv * tb);
-    const int64_t steps = (max_n + ATT_CH - 1) / ATT_CH;
-    if (nsplit > steps) nsplit = steps;
-    if (nsplit < 1) nsplit = 1;
-    int64_t span = ((steps + nsplit - 1) / nsplit) * ATT_CH;
-    nsplit = (max_n + span - 1) / span;
-    if (nsplit > 65535 || span > 0x7FFFFFFF) {
-        LOG("%s: kv range too long", op);
-        return 0;
-    }
     if (!need_batch(op)) return 0;
-    const size_t part_bytes = (size_t)tb * (size_t)H * (size_t)nsplit * (size_t)(Dh + 2) * 8;
-    double *part = (double *)scratch(part_bytes, op);
-    if (!part) return 0;
     if (!prep_in_r(q, 0, qb, op) || !prep_in_r(k, 0, kvb, op) || !prep_in_r(v, 0, kvb, op) ||
         !prep_in_r(rel_logits, 0, rlb, op) || !prep_out(attn_out, op))
         return 0;
-    int32_t H32 = (int32_t)H, Hkv32 = (int32_t)Hkv, Dh32 = (int32_t)Dh, R32 = (int32_t)rel_extent;
-    int32_t ns32 = (int32_t)nsplit, span32 = (int32_t)span;
-    int64_t qpb = q_pos_base, kvd = kv_dim;
-    float ihd = inv_head_dim;
-    for (int64_t t0 = 0; t0 < T; t0 += ATT_TB) {
-        const int64_t nt = T - t0 < ATT_TB ? T - t0 : ATT_TB;
-        AttnTok tok;
-        memset(&tok, 0, sizeof tok);
-        for (int64_t i = 0; i < nt; i++) {
-            tok.lo[i] = (int32_t)kv_lo[t0 + i];
-            tok.hi[i] = (int32_t)kv_hi[t0 + i];
-            tok.tau[i] = tau[t0 + i];
-        }
-        int32_t t032 = (int32_t)t0;
-        void *a_p[] = { &q->dev, &k->dev, &v->dev, &rel_logits->dev, &tok, &t032, &H32, &Hkv32, &Dh32, &R32, &qpb,
-                        &kvd, &ihd, &ns32, &span32, &part };
-        if (!launch3(K_ATTN_PARTIAL, (unsigned)nsplit, (unsigned)Hkv, (unsigned)nt, 256, 0, a_p, op)) return 0;
-        void *a_c[] = { &part, &tok, &t032, &H32, &Dh32, &ns32, &span32, &attn_out->dev };
-        if (!launch2(K_ATTN_COMBINE, (unsigned)H, (unsigned)nt, 128, 0, a_c, op)) return 0;
+    for (int64_t t0 = 0; t0 < T; t0 += ATT_TMAX) {
+        AttnArgs a;
+        memset(&a, 0, sizeof a);
+        a.q = (const float *)q->dev + t0 * H * Dh;
+        a.k = (const float *)k->dev;
+        a.v = (const float *)v->dev;
+        a.rel = (const float *)rel_logits->dev + t0 * H * rel_extent;
+        a.out = (float *)attn_out->dev + t0 * H * Dh;
+        a.q_pos_base = q_pos_base + t0;
+        a.kv_dim = kv_dim;
+        a.T = (int32_t)(T - t0 < ATT_TMAX ? T - t0 : ATT_TMAX);
+        a.H = (int32_t)H;
+        a.Hkv = (int32_t)Hkv;
+        a.Dh = (int32_t)Dh;
+        a.R = (int32_t)rel_extent;
+        a.inv_head_dim = inv_head_dim;
+        if (!attn_launch(op, a, t0, kv_lo, kv_hi, tau)) return 0;
     }
     return 1;
 }
@@ -1436,7 +1519,6 @@ int sepia_hip_set_option(const char *name, int value) {
  * and Q3_K 7, Q4_K 9). nw = C * P waves: P parts split each item's quads, C
  * items run side by side; every wave's ring holds S = min(4, ring / Wp KB)
  * steps in flight. */
-#define MQ_CUS 256                  /* MI355X compute units */
 #define MQ_ZERO 768
 typedef struct {
     int32_t P, ring, xraw, orings, conv, nw;   /* as struct MqGeo in kernels/mq.h */

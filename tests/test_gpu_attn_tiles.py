@@ -1,0 +1,83 @@
+"""The matrix-core attention kernels at the sizes where their tiling can go
+wrong: head dims off the 16-wide steps, query heads per kv head that do not
+divide a tile, token counts at the edges of the 16- and 64-row tiles and of
+the bounds in the kernel arguments (64, then 256 a launch), kv ranges off the
+16- and 32-row steps and split over workgroups, and NaN or infinite v rows
+that only some of a tile's rows see. All against the oracle's restatement of
+the reference's loop (src/sepia.c:1203-1247)."""
+import numpy as np
+import pytest
+
+from sepia_amd import hip
+from test_gpu_attn import banded
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    return hip.Device()
+
+
+def make(rng, T, H, Hkv, Dh, R, n, window, extra=0):
+    kv_dim = Hkv * Dh + extra
+    q = (rng.standard_normal(T * H * Dh) * 0.5).astype(np.float32)
+    k = (rng.standard_normal(n * kv_dim) * 0.5).astype(np.float32)
+    v = (rng.standard_normal(n * kv_dim) * 0.5).astype(np.float32)
+    rl = (rng.standard_normal(T * H * R) * 0.5).astype(np.float32)
+    qpb = n - T
+    hi = [qpb + t for t in range(T)]
+    lo = [max(0, h - window + 1) for h in hi]
+    tau = np.linspace(1.0, 1.5, T).astype(np.float32)
+    return q, k, v, rl, lo, hi, tau, T, H, Hkv, Dh, R, qpb, kv_dim
+
+
+def check(dev, orc, args):
+    got = banded(dev, *args)
+    want = orc.banded_attn(*args, 1.0 / args[10])
+    # f32 scores of at most a few units: each weight is within about 1e-6
+    # relative, and the weighted sums and their quotient are double
+    fin = np.isfinite(want)
+    assert np.array_equal(fin, np.isfinite(got)) and np.array_equal(np.isnan(want), np.isnan(got))
+    assert np.array_equal(got[~fin & ~np.isnan(want)], want[~fin & ~np.isnan(want)])
+    err = np.abs(got[fin].astype(np.float64) - want[fin])
+    assert not fin.any() or err.max() <= 5e-6 * np.abs(want[fin]).max()
+
+
+# (T, H, Hkv, Dh, R, kv positions, window): one 16-row tile and its edges
+# (rows = T H / Hkv = 16, 17, 32), the 64-row kernel from 33 rows, its tile
+# edges (64, 65, 128 rows), bounds in the arguments up to 64 tokens and in
+# scratch beyond (65, 256, 257), kv ranges around the steps and long ones
+SHAPES = [
+    (1, 8, 8, 128, 16, 1, 1), (1, 8, 8, 128, 16, 17, 17), (1, 64, 8, 128, 1024, 4097, 4097), (2, 8, 1, 128, 7, 40, 40),
+    (17, 4, 4, 128, 33, 80, 64), (4, 16, 2, 128, 100, 200, 31), (33, 2, 2, 128, 64, 97, 50), (11, 9, 3, 36, 20, 70, 33),
+    (4, 16, 1, 100, 300, 333, 333), (5, 16, 1, 4, 8, 64, 64), (3, 48, 3, 124, 9, 150, 20), (64, 3, 3, 64, 40, 65, 32),
+    (65, 4, 1, 128, 128, 400, 100), (256, 2, 2, 128, 30, 300, 70), (257, 4, 4, 20, 12, 290, 290), (66, 7, 1, 8, 5, 99, 40),
+]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_shapes(dev, orc, shape):
+    T, H, Hkv, Dh, R, n, window = shape
+    check(dev, orc, make(np.random.default_rng(T * 31 + n), T, H, Hkv, Dh, R, n, window, extra=4 * (T % 3)))
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf], ids=["nan", "inf", "-inf"])
+@pytest.mark.parametrize("T,H,Hkv,n,window", [(2, 16, 2, 60, 40), (1, 8, 1, 300, 300), (40, 8, 4, 200, 64),
+                                              (70, 8, 2, 150, 150)], ids=str)
+def test_nonfinite_rows(dev, orc, bad, T, H, Hkv, n, window):
+    """A bad v element reaches exactly the tokens whose range holds its row (a
+    matrix op would also give 0 * bad to the tile's other tokens), a bad k
+    element exactly the scores it enters; neighbours outside every range stay
+    unread."""
+    rng = np.random.default_rng(T + n)
+    args = make(rng, T, H, Hkv, 128, 64, n, window)
+    k, v, kv_dim = args[1], args[2], args[13]
+    first = args[4][0]
+    for row in {n - 1, n - 1 - T // 2, first, max(0, first - 1), min(n - 1, first + T // 2)}:
+        v[row * kv_dim + 5 * (row % 20)] = bad
+    check(dev, orc, args)
+    args = make(rng, T, H, Hkv, 128, 64, n, window)
+    args[1][(n - 1) * args[13] + 3] = bad
+    args[1][max(0, args[4][0] - 1) * args[13]] = bad
+    check(dev, orc, args)
