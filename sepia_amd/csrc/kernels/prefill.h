@@ -12,11 +12,14 @@
 //   sepia_pf_select   one wave per token: idx[T][topk], w[T][topk + n_shared]
 //   sepia_pf_group    one workgroup: the (token, slot) pairs p = t * n_sel + k
 //                     sorted by expert (shared expert s is expert
-//                     n_routed + s) and cut into units of <= 32 pairs
+//                     n_routed + s) and cut into units of <= 32 pairs (f16
+//                     path: 64)
 //   projections       a layer whose six projections are all Q2_K, Q3_K or
 //                     Q4_K runs them on the int8 matrix cores (prefill_q.h:
-//                     sepia_pf_quant, sepia_pf_gateup_q, sepia_pf_down_q);
-//                     any other layer on the bf16 matrix cores here:
+//                     sepia_pf_quant, sepia_pf_gateup_q, sepia_pf_down_q); any
+//                     other layer on the f16 ones (prefill_h.h:
+//                     sepia_ph_quant, sepia_ph_gateup, sepia_ph_down); layers
+//                     with rows at 2-byte offsets on the bf16 ones here:
 //     sepia_pf_split    x as bf16 hi / lo
 //     sepia_pf_gateup   per (32-row tile, unit): h[p][.] = silu(g) * u (bf16 hi / lo)
 //     sepia_pf_down     per (64-row tile, unit): yp[p][.] = down_e . h[p]
@@ -41,23 +44,26 @@ typedef float pf_f32x4 __attribute__((ext_vector_type(4)));
 #define PF_MT 32     // pairs per unit (two 16-row M tiles)
 
 // (row slice x, unit y) of this workgroup in a (slices x units) launch of
-// a unit kernel. The hardware deals consecutive workgroup ids to the 8 XCDs
-// in turn; when the unit count is a multiple of 8 the units are dealt to
-// the XCDs the same way (XCD c runs units c, c + 8, ..., each over all its
-// slices in a row), so the workgroups of a unit, which all read that unit's
-// activation rows, share one XCD's L2. The f16 kernels use it (their C5
-// layer in the real formats: 3.79 -> 3.02 ms); the int8 ones measured no
-// better with it (1.90 -> 1.93 ms) and keep the launch order.
+// a unit kernel, n_units of whose units exist. The hardware deals consecutive
+// workgroup ids to the 8 XCDs in turn; with many units they are dealt to the
+// XCDs the same way (XCD c runs units c, c + 8, ..., each over all its slices
+// in a row), so the workgroups of a unit, which all read that unit's
+// activation rows, share one XCD's L2 (the f16 kernels' layer of 512 tokens
+// in the real formats: 3.79 -> 3.02 ms when it came in). A few units would
+// leave some XCDs one more each than others (51 units of 24 slices on 32 CUs
+// an XCD: 6 rounds where 5 do; 9 tokens: gate/up 352 -> 328 us), and their
+// rows are few:
+// they keep the launch order, as the int8 kernels do, which measured no better with the dealing (1.90 -> 1.93 ms).
+#define PF_DEAL_UNITS 128
 struct PfSlot {
     int32_t x, y;
 };
-__device__ __forceinline__ PfSlot pf_slot() {
+__device__ __forceinline__ PfSlot pf_slot(int32_t n_units) {
     const uint32_t gx = gridDim.x;
-    if (gridDim.y % 8u) return PfSlot{(int32_t)blockIdx.x, (int32_t)blockIdx.y};
+    if (gridDim.y % 8u || n_units < PF_DEAL_UNITS) return PfSlot{(int32_t)blockIdx.x, (int32_t)blockIdx.y};
     const uint32_t lid = blockIdx.y * gx + blockIdx.x, k = lid >> 3;
     return PfSlot{(int32_t)(k % gx), (int32_t)(8u * (k / gx) + (lid & 7u))};
 }
-
 
 // ------------------------------------------------------------- router ----
 // logits[t][r] = sum_k x[t][k] * Rw[r][k]: 32 tokens x 32 rows per
@@ -182,9 +188,9 @@ extern "C" __global__ __launch_bounds__(64) void sepia_pf_select(const float *__
 // n_routed + (k - topk) after. list[] holds the pairs grouped by expert
 // (ascending expert; within an expert in arrival order, which does not
 // affect any result), units[u] = {expert, first list position, count <=
-// PF_MT}, n_units[0] their number. E = n_routed + n_shared <= 1088.
+// um}, n_units[0] their number. E = n_routed + n_shared <= 1088.
 extern "C" __global__ __launch_bounds__(1024) void sepia_pf_group(const int32_t *__restrict__ idx, int64_t T,
-                                                                  int32_t n_routed, int32_t n_shared, int32_t topk,
+                                                                  int32_t n_routed, int32_t n_shared, int32_t topk, int32_t um,
                                                                   int32_t *__restrict__ list,
                                                                   int32_t *__restrict__ units,
                                                                   int32_t *__restrict__ n_units) {
@@ -209,7 +215,7 @@ extern "C" __global__ __launch_bounds__(1024) void sepia_pf_group(const int32_t 
             off[e] = a;
             uoff[e] = u;
             a += cnt[e];
-            u += (cnt[e] + PF_MT - 1) / PF_MT;
+            u += (cnt[e] + um - 1) / um;
         }
         off[E] = a;
         uoff[E] = u;
@@ -221,11 +227,11 @@ extern "C" __global__ __launch_bounds__(1024) void sepia_pf_group(const int32_t 
         list[off[e] + atomicAdd(&fill[e], 1)] = (int32_t)p;
     }
     for (int e = threadIdx.x; e < E; e += blockDim.x) {
-        for (int j = 0; j < (cnt[e] + PF_MT - 1) / PF_MT; j++) {
+        for (int j = 0; j < (cnt[e] + um - 1) / um; j++) {
             int32_t *un = units + 3 * (uoff[e] + j);
             un[0] = e;
-            un[1] = off[e] + PF_MT * j;
-            un[2] = cnt[e] - PF_MT * j < PF_MT ? cnt[e] - PF_MT * j : PF_MT;
+            un[1] = off[e] + um * j;
+            un[2] = cnt[e] - um * j < um ? cnt[e] - um * j : um;
         }
     }
 }

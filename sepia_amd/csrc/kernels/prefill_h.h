@@ -1,8 +1,7 @@
-// prefill_h.h -- the prefill MoE projections of the real checkpoint's
-// formats (IQ2_XS, IQ3_XXS, IQ4_XS routed; Q5_K, Q6_K, Q8_0 shared) on the
-// f16 matrix cores: the batched layer of prefill.h with the same grouping,
-// units and combine, for layers whose six projections all have one of
-// these formats.
+// prefill_h.h -- the prefill MoE projections on the f16 matrix cores: the
+// batched layer of prefill.h with the same grouping and combine, for layers
+// in the real checkpoint's formats (IQ2_XS, IQ3_XXS, IQ4_XS routed; Q5_K,
+// Q6_K, Q8_0 shared) and for mixes of those with Q2_K, Q3_K and Q4_K.
 //
 // Activations (x per token for gate/up, h per pair for down) travel as "PH"
 // rows: per row a power-of-two scale s > max|v| (s = 1 for a zero row,
@@ -10,9 +9,10 @@
 // output of the row non-finite), and per column v' = v / s (|v'| < 1,
 // exact) as two f16 planes, hi = f16(v') and lo = f16(v' - hi): together
 // within 2^-23 of v' (lo's rounding, or the f16 subnormal spacing 2^-24).
-// A 256-column block of a row is a 1056-byte record: hi (256 f16, column
-// order), lo (256 f16), then the eight 32-column sums of v' (f32, column
-// order) that the Q5_K min terms use.
+// 128 columns of a row are a 576-byte record: hi (128 f16, column order),
+// lo (128 f16), then four 16-byte groups, one per 32 columns, for the min
+// terms of Q2_K, Q4_K and Q5_K: the two 16-column sums of v', each as three
+// f16 (together within 2^-25 of the f32 sum), and two zeros.
 //
 // Weights enter v_mfma_f32_16x16x32_f16 as exact f16 integer codes, decoded
 // from the raw blocks in registers (the products hi * code and lo * code are
@@ -25,9 +25,12 @@
 //   IQ3_XXS  code = +-grid * (2 s + 1) * 2^-14, 4-bit s per 32 weights
 //            (|code| <= 62 * 31 * 2^-14), sum w x = d C 2^14 / 4
 //            (quants.c:203-226)
-//   Q5_K     code = q * sc, 6-bit sc per 32 (<= 31 * 63);
-//            sum w x = d C - dmin sum_j m_j S_j, S_j the record's sums
-//            (quants.c:127-151)
+//   Q4_K     code = q * sc, 6-bit sc per 32 (<= 15 * 63); sum w x = d C -
+//   Q5_K     dmin sum_j m_j S_j (Q5_K: code <= 31 * 63), the min terms as one
+//            more matrix op: the records' sums against the mins
+//            (quants.c:104-151)
+//   Q2_K     the same with 4-bit sc and m per 16 weights (<= 3 * 15)
+//   Q3_K     code = (q - 4) * (sc - 32), sc per 16; sum w x = d C
 //   Q6_K     int8 sc per 16 weights split as 16 a + b (b in 0..15):
 //            codes (q - 32) b and (q - 32) a, sum w x = d (C_b + 16 C_a)
 //            (quants.c:153-177)
@@ -46,56 +49,68 @@
 // subnormal as such: f16 denormals are on in the kernels' default FP mode,
 // and a flush would zero every IQ code, which every IQ parity case shows.)
 //
-// Workgroup: one unit (<= 32 pairs of one expert) x R weight rows (R = 256:
-// gate/up 128 gate + the same 128 up rows; R = 128 for the formats whose
-// staged blocks are too large for 256 rows: Q6_K, Q8_0), 16 waves; wave
-// w < R / (16 NT) computes 16 NT rows (NT N tiles: 2 for the 256-row
-// formats, so each activation read feeds two, else 1) x the unit's one or
-// two 16-pair M tiles; the other waves only stage records. Records are double-buffered; weights SW-buffered, and
-// a stepping wave stages exactly the weight rows it decodes (each row's block from
-// the 4-byte boundary at or below its start, PW 16-byte pieces), so only
-// the records need the per-block barrier.
+// Workgroup: one unit (<= 64 pairs of one expert, MT = 1..4 M tiles of 16) x
+// 8 waves; a wave computes two N tiles of 16 weight rows (gate/up: the same
+// rows of gate and of up, so silu(gate) * up needs no exchange) x the unit's
+// M tiles. A wave's weights come G blocks (256 columns) of its rows at a time,
+// as whole 16-byte pieces along the rows, to registers a group ahead and from
+// there to its own part of LDS, where its lanes read what they decode. The
+// unit's records, half a block at a time, go through registers to a double
+// buffer in LDS that all waves read, one barrier a half.
+//
+// What bounds it: the LDS pipe (activation reads, codebook gathers at 2-3
+// times their conflict-free cost) and the latency between its results and
+// the matrix ops, at two waves a SIMD. Measured, gate/up + down at hidden 6144,
+// inter 3072, 256 experts, IQ2_XS / IQ3_XXS with Q5_K / Q6_K shared: 1999
+// tokens 3.30 + 1.87 ms (units of 64 pairs; 4.36 + 2.94 ms with units of 32
+// whose 16 waves staged single blocks by LDS DMA), 512 tokens 1.30 + 0.77 ms
+// (1.57 + 1.09), 9 tokens 328 + 203 us (363 + 238). Loads alone take 125 us
+// of the 328: a wave instruction that reads whole pieces along a row touches
+// each line once; lanes loading just what they decode took 369 us for the
+// same bytes. Four N tiles a wave for the larger units (half the activation
+// reads, groups of one block) took 3.35 + 1.97 ms; all of a half's table
+// reads at once 397 us for 9 tokens; units of up to 16 pairs in a launch of
+// their own with two workgroups a CU 334 + 203 us there, but 538 + 1044 us
+// for the two gate/up launches of 512 tokens.
 #pragma once
 #include "prefill_q.h"
 
-#define PH_REC 1056                    // bytes of a 256-column PH record
-#define PH_AP 66                       // its 16-byte pieces (2 mod 4: no LDS bank conflicts)
-#define PH_ABYTES (PF_MT * PH_REC)     // a record stage: the unit's 32 rows
-#define PH_WAVES 16                    // waves of a workgroup
+#define PH_UM 64                       // pairs per unit
+#define PH_REC 576                     // bytes of a 128-column PH record
+#define PH_LREC 608                    // a staged record (38 16-byte pieces, 2 mod 4: no LDS bank conflicts)
+#define PH_WAVES 8                     // waves of a workgroup
 
 typedef _Float16 ph_h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 ph_h8 __attribute__((ext_vector_type(8)));
 typedef uint32_t ph_u4 __attribute__((ext_vector_type(4)));
 
-// BB: block bytes (256 columns); PW: 16-byte pieces of a staged row (the
-// block from the 4-byte boundary at or below its start, at most 2 bytes
-// earlier); SW: weight stages; R: weight rows of a workgroup; NT: 16-row N
-// tiles of a stepping wave; STEP: scale per 32-column step applied in f32
-// (else once per block).
+// BB: block bytes (256 columns); QN: dwords of a lane's half block, HN: of
+// what it needs of the block besides; G, GL: blocks of a weight group for
+// units of up to two M tiles and of more (what the LDS holds); STEP: scale
+// per 32-column step applied in f32 (else once per block); MIN: min terms.
 template <int T> struct PhFmt;
-template <> struct PhFmt<ST_IQ2_XS> { static constexpr int BB = 74, PW = 6, SW = 3, R = 256, NT = 2; static constexpr bool STEP = false; };
-template <> struct PhFmt<ST_IQ3_XXS> { static constexpr int BB = 98, PW = 10, SW = 2, R = 256, NT = 2; static constexpr bool STEP = false; };
-template <> struct PhFmt<ST_IQ4_XS> { static constexpr int BB = 136, PW = 10, SW = 2, R = 256, NT = 2; static constexpr bool STEP = true; };
-template <> struct PhFmt<ST_Q5_K> { static constexpr int BB = 176, PW = 11, SW = 2, R = 256, NT = 2; static constexpr bool STEP = false; };
-template <> struct PhFmt<ST_Q6_K> { static constexpr int BB = 210, PW = 14, SW = 2, R = 128, NT = 1; static constexpr bool STEP = false; };
-template <> struct PhFmt<ST_Q8_0> { static constexpr int BB = 272, PW = 17, SW = 2, R = 128, NT = 1; static constexpr bool STEP = true; };
+template <> struct PhFmt<ST_Q2_K> { static constexpr int BB = 84, QN = 4, HN = 1, G = 4, GL = 2; static constexpr bool STEP = false, MIN = true; };
+template <> struct PhFmt<ST_Q3_K> { static constexpr int BB = 110, QN = 2, HN = 6, G = 4, GL = 2; static constexpr bool STEP = false, MIN = false; };
+template <> struct PhFmt<ST_Q4_K> { static constexpr int BB = 144, QN = 4, HN = 4, G = 2, GL = 2; static constexpr bool STEP = false, MIN = true; };
+template <> struct PhFmt<ST_Q5_K> { static constexpr int BB = 176, QN = 4, HN = 6, G = 2, GL = 1; static constexpr bool STEP = false, MIN = true; };
+template <> struct PhFmt<ST_Q6_K> { static constexpr int BB = 210, QN = 8, HN = 1, G = 2, GL = 1; static constexpr bool STEP = false, MIN = false; };
+template <> struct PhFmt<ST_IQ2_XS> { static constexpr int BB = 74, QN = 3, HN = 1, G = 4, GL = 2; static constexpr bool STEP = false, MIN = false; };
+template <> struct PhFmt<ST_IQ3_XXS> { static constexpr int BB = 98, QN = 3, HN = 1, G = 4, GL = 2; static constexpr bool STEP = false, MIN = false; };
+template <> struct PhFmt<ST_IQ4_XS> { static constexpr int BB = 136, QN = 8, HN = 2, G = 2, GL = 2; static constexpr bool STEP = true, MIN = false; };
+template <> struct PhFmt<ST_Q8_0> { static constexpr int BB = 272, QN = 12, HN = 1, G = 1, GL = 1; static constexpr bool STEP = true, MIN = false; };
 
-// LDS: [record stages 2 x PH_ABYTES][weight stages SW x R x PW x 16]
-//      [tables: IQ2_XS grid 4 KB / IQ3_XXS grid 1 KB, then 128 x 8 sign
-//       bytes][... row tables at PQ_LDS_TOP]
-template <int T> struct PhLds {
-    static constexpr uint32_t W = (uint32_t)PhFmt<T>::R * PhFmt<T>::PW * 16;
-    static constexpr uint32_t TAB = 2 * PH_ABYTES + PhFmt<T>::SW * W;
-    static constexpr uint32_t GRID = T == ST_IQ2_XS ? 4096u : T == ST_IQ3_XXS ? 1024u : 0u;
-    static constexpr uint32_t SIGNS = TAB + GRID;
-    static constexpr uint32_t END = SIGNS + (GRID ? 1024u : 0u);
-    static_assert(END <= PQ_LDS_TOP, "LDS of a PH projection");
-};
+// LDS: [record stages 2 x 16 MT x PH_LREC][weight groups: 8 waves x 2 tiles
+// x 16 rows x PW pieces] ... [IQ2_XS grid 4 KB / IQ3_XXS grid 1 KB][128 x 8
+// sign bytes][row tables]
+#define PH_LDS_BYTES 163840
+#define PH_O_ROWS (PH_LDS_BYTES - 16 * PH_UM)
+#define PH_O_SIGNS (PH_O_ROWS - 1024)
+#define PH_O_TAB (PH_O_SIGNS - 4096)
 
 // --------------------------------------------------------- rows -> PH ----
 // One workgroup per row: src row r (K floats at src + r * ld) into its
 // records at rec + r * ldr and its scale at scale[r]. Thread i converts the
-// 32-column groups i, i + 256, ...
+// 16-column groups i, i + 256, ...
 extern "C" __global__ __launch_bounds__(256) void sepia_ph_quant(const float *__restrict__ src, int64_t ld,
                                                                  int64_t K, uint8_t *__restrict__ rec, int64_t ldr,
                                                                  float *__restrict__ scale) {
@@ -120,113 +135,40 @@ extern "C" __global__ __launch_bounds__(256) void sepia_ph_quant(const float *__
     const float s = !fin ? INFINITY : ldexpf(1.0f, e), inv = fin ? ldexpf(1.0f, -e) : 0.0f;
     if (threadIdx.x == 0) scale[r] = s;
     uint8_t *out = rec + r * ldr;
-    for (int64_t gi = threadIdx.x; gi < K / 32; gi += 256) {
-        const float4 *x4 = (const float4 *)(row + 32 * gi);
+    for (int64_t gi = threadIdx.x; gi < K / 16; gi += 256) {
+        const float4 *x4 = (const float4 *)(row + 16 * gi);
         uint8_t *blk = out + (gi >> 3) * PH_REC;
         const int j = (int)(gi & 7);
         float sum = 0.0f;
+        _Float16 h[16], l[16];
 #pragma unroll
-        for (int c = 0; c < 8; c++) {
+        for (int c = 0; c < 4; c++) {
             const float4 t = x4[c];
             const float a[4] = {t.x * inv, t.y * inv, t.z * inv, t.w * inv};
-            _Float16 h[4], l[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 sum += a[i];
-                h[i] = (_Float16)a[i];
-                l[i] = (_Float16)(a[i] - (float)h[i]);
+                h[4 * c + i] = (_Float16)a[i];
+                l[4 * c + i] = (_Float16)(a[i] - (float)h[4 * c + i]);
             }
-            *(uint2 *)(blk + 64 * j + 8 * c) = *(const uint2 *)h;
-            *(uint2 *)(blk + 512 + 64 * j + 8 * c) = *(const uint2 *)l;
         }
-        *(float *)(blk + 1024 + 4 * j) = fin ? sum : 0.0f;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            *(uint4 *)(blk + 32 * j + 16 * i) = *(const uint4 *)(h + 8 * i);
+            *(uint4 *)(blk + 256 + 32 * j + 16 * i) = *(const uint4 *)(l + 8 * i);
+        }
+        sum = fin ? sum : 0.0f;
+        const _Float16 s0 = (_Float16)sum, s1 = (_Float16)(sum - (float)s0),
+                       s2 = (_Float16)(sum - (float)s0 - (float)s1);
+        _Float16 *sp = (_Float16 *)(blk + 512 + 16 * (j >> 1)) + 3 * (j & 1);
+        sp[0] = s0;
+        sp[1] = s1;
+        sp[2] = s2;
+        if (j & 1) sp[3] = sp[4] = (_Float16)0.0f;
     }
 }
-
-// ------------------------------------------------------------- staging --
-// Record pieces: the unit's records of a block (its nv <= 32 pairs, 66
-// pieces each, record m at 1056 m) by up to 33 wave instructions over the 16
-// waves. Weight pieces:
-// stepping wave w (w < R / RW, RW = 16 NT) stages its RW rows, piece c of
-// row k at 16 (PW (RW w + k) + c); a piece that starts past the block's bytes (plus
-// the 2 of the 4-byte alignment) takes piece 0's bytes again. The last
-// piece that holds block bytes may run up to 14 bytes past the block: into
-// the row's next block, the next row, or, after a matrix's last row, the
-// 256 bytes every device buffer of the library carries past its data
-// (dev_bytes in sepia_hip.c).
-template <int T, bool GU>
-struct PhDma {
-    static constexpr int BB = PhFmt<T>::BB, PW = PhFmt<T>::PW, R = PhFmt<T>::R, RW = 16 * PhFmt<T>::NT, AW = R / RW;
-    static constexpr int NA = (PF_MT * PH_AP + 63) / 64, KA = (NA + PH_WAVES - 1) / PH_WAVES;
-    static constexpr int NW = RW * PW, KW = (NW + 63) / 64;   // a stepping wave's weight pieces and instructions
-    uint32_t a[KA];            // record piece offsets at block 0
-    uint32_t r[KW], c16[KW];   // row offset from the matrix base; offset of the lane's piece in the window
-    bool aon[KA], won[KW];
-    // nr: the records the unit's M tiles read (its pairs; the rest of the
-    // stage is not staged, and the M tile rows past the pairs are discarded)
-    __device__ __forceinline__ void init(const uint32_t *roff, uint64_t row_bytes, int64_t r0, int nr) {
-        const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-#pragma unroll
-        for (int k = 0; k < KA; k++) {
-            const int q = 64 * (w + PH_WAVES * k) + lane, m = q / PH_AP, c = q - m * PH_AP;
-            aon[k] = w + PH_WAVES * k < NA && q < PF_MT * PH_AP && m < nr;
-            a[k] = aon[k] ? roff[m] + 16u * (uint32_t)c : 0u;
-        }
-        // stepping waves 0 .. AW - 1 take RW rows each; GU: the first half
-        // the gate rows, the second half the same up rows
-        const bool on = w < AW;
-        const int64_t rw0 = r0 + (int64_t)(RW * (GU ? w % (AW / 2) : w));
-#pragma unroll
-        for (int k = 0; k < KW; k++) {
-            const int q = 64 * k + lane, kr = q / PW, c = q - kr * PW;
-            won[k] = on && q < NW;
-            r[k] = won[k] ? (uint32_t)((uint64_t)(rw0 + kr) * row_bytes) : 0u;
-            c16[k] = 16 * c < BB + 2 ? 16u * (uint32_t)c : 0u;
-        }
-    }
-    __device__ __forceinline__ void issue_a(int64_t b, uint8_t *As, const uint8_t *rec) const {
-        const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-        const uint32_t ab = (uint32_t)b * PH_REC;
-#pragma unroll
-        for (int k = 0; k < KA; k++) {
-            const int jj = w + PH_WAVES * k;
-            if (jj < NA && aon[k]) pf_dma16(rec, a[k] + ab, pf_lds(As + 1024 * jj));
-        }
-    }
-    // a stepping wave's weight instructions of one block (other waves: none)
-    __device__ __forceinline__ void issue_w(int64_t b, uint8_t *Ws, const uint8_t *Wm) const {
-        const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-        if (w >= AW) return;
-        const uint32_t wb = (uint32_t)b * BB;
-        uint8_t *dst = Ws + 16 * NW * w;
-#pragma unroll
-        for (int k = 0; k < KW; k++)
-            if (won[k]) pf_dma16(Wm, ((r[k] + wb) & ~3u) + c16[k], pf_lds(dst + 1024 * k));
-    }
-};
 
 // ------------------------------------------------------------- decoders --
-typedef const __attribute__((address_space(3))) uint32_t ph_lds_u32;
-typedef const __attribute__((address_space(3))) uint16_t ph_lds_u16;
-typedef const __attribute__((address_space(3))) uint8_t ph_lds_u8;
-__device__ __forceinline__ uint32_t ph_u8(const uint8_t *p) { return *(ph_lds_u8 *)(size_t)pf_lds(p); }
-__device__ __forceinline__ uint32_t ph_u16(const uint8_t *p) { return *(ph_lds_u16 *)(size_t)pf_lds(p); }
-__device__ __forceinline__ float ph_h2f(const uint8_t *p) { return f16_bits_to_f32(ph_u16(p)); }
-// 4 bytes at a 2-byte-aligned LDS address: the two aligned dwords around
-// it, funnel-shifted
-__device__ __forceinline__ uint32_t ph_u32(const uint8_t *p) {
-    const uint32_t a = pf_lds(p), a4 = a & ~3u;
-    const uint32_t lo = *(ph_lds_u32 *)(size_t)a4, hi = *(ph_lds_u32 *)(size_t)(a4 + 4u);
-    return __builtin_amdgcn_alignbit(hi, lo, 8u * (a & 3u));
-}
-// 8 bytes at a 2-byte-aligned LDS address
-__device__ __forceinline__ uint2 ph_u64(const uint8_t *p) {
-    const uint32_t a = pf_lds(p), a4 = a & ~3u, sh = 8u * (a & 3u);
-    const uint32_t d0 = *(ph_lds_u32 *)(size_t)a4, d1 = *(ph_lds_u32 *)(size_t)(a4 + 4u),
-                   d2 = *(ph_lds_u32 *)(size_t)(a4 + 8u);
-    return make_uint2(__builtin_amdgcn_alignbit(d1, d0, sh), __builtin_amdgcn_alignbit(d2, d1, sh));
-}
-
 // Bytes 0, 1 (sel 0x04010400) or 2, 3 (sel 0x04030402) of v as the halves
 // 0x64bb: 1024 + b, exact.
 __device__ __forceinline__ ph_h2 ph_bias2(uint32_t v, uint32_t sel) {
@@ -277,11 +219,11 @@ __device__ __forceinline__ ph_h8 ph_codes_iq(uint2 g, uint2 sg, ph_h2 s2) {
 template <int T>
 __device__ __forceinline__ void ph_fill_tables(uint8_t *smem) {
     if constexpr (T == ST_IQ2_XS) {
-        for (int i = threadIdx.x; i < 512; i += blockDim.x) ((uint64_t *)(smem + PhLds<T>::TAB))[i] = c_iq2xs_grid[i];
-        ph_fill_signs(smem + PhLds<T>::SIGNS);
+        for (int i = threadIdx.x; i < 512; i += blockDim.x) ((uint64_t *)(smem + PH_O_TAB))[i] = c_iq2xs_grid[i];
+        ph_fill_signs(smem + PH_O_SIGNS);
     } else if constexpr (T == ST_IQ3_XXS) {
-        for (int i = threadIdx.x; i < 256; i += blockDim.x) ((uint32_t *)(smem + PhLds<T>::TAB))[i] = c_iq3xxs_grid[i];
-        ph_fill_signs(smem + PhLds<T>::SIGNS);
+        for (int i = threadIdx.x; i < 256; i += blockDim.x) ((uint32_t *)(smem + PH_O_TAB))[i] = c_iq3xxs_grid[i];
+        ph_fill_signs(smem + PH_O_SIGNS);
     }
 }
 
@@ -299,320 +241,513 @@ __device__ __forceinline__ uint32_t ph_iq4_levels(uint32_t c) {
     return __builtin_amdgcn_perm(hi, lo, ((c >> 1) & 0x04040404u) | 0x03020100u);
 }
 
-// Q5_K's 6-bit scale and min of sub-block j from the 12 scale bytes at p
-// (the packing of get_scale_min_k4, src/quants.c:96-102).
-__device__ __forceinline__ uint32_t k_scale_6(const uint8_t *p, int j) {
-    return j < 4 ? ph_u8(p + j) & 63u : (ph_u8(p + j + 4) & 15u) | ((ph_u8(p + j - 4) >> 6) << 4);
-}
-__device__ __forceinline__ uint32_t k_min_6(const uint8_t *p, int j) {
-    return j < 4 ? ph_u8(p + j + 4) & 63u : (ph_u8(p + j + 4) >> 4) | ((ph_u8(p + j) >> 6) << 4);
+// N dwords of a staged row at byte p. M: whether p is 2 bytes past a dword
+// (else at one): two aligned dwords around each, funnel-shifted.
+template <int N, bool M>
+__device__ __forceinline__ void ph_gld(const uint8_t *p, uint32_t *q) {
+    const uint32_t at = pf_lds(p) - (M ? 2u : 0u);
+    uint32_t d[N + 1];
+#pragma unroll
+    for (int i = 0; i < N + (M ? 1 : 0); i++)
+        d[i] = *(const __attribute__((address_space(3))) uint32_t *)(size_t)(at + 4u * (uint32_t)i);
+#pragma unroll
+    for (int i = 0; i < N; i++) q[i] = M ? __builtin_amdgcn_alignbit(d[i + 1], d[i], 16) : d[i];
 }
 
-// What a lane decodes for K step s (columns 32 s .. 32 s + 31 of the block;
-// lane group g takes columns 32 s + 8 g .. + 7) of its row's block: the 8
-// codes (two operands for Q6_K) and, for the STEP formats, the step's scale.
+// What lane group g needs of the block at p besides the half's codes. M: the
+// block starts 2 bytes past a dword.
+template <int T, bool M>
+__device__ __forceinline__ void ph_load_head(const uint8_t *p, int g, uint32_t *h) {
+    if constexpr (T == ST_Q2_K) {
+        ph_gld<1, M>(p + 80, h);   // d, dmin
+    } else if constexpr (T == ST_Q3_K) {
+        ph_gld<2, M>(p + 8 * g, h);       // hmask bytes 8 g ..
+        ph_gld<3, M>(p + 96, h + 2);      // scales: low nibbles, then the high bits
+        ph_gld<1, !M>(p + 106, h + 5);    // d in the high half
+    } else if constexpr (T == ST_Q4_K) {
+        ph_gld<4, M>(p, h);   // d, dmin, 12 scale bytes
+    } else if constexpr (T == ST_Q5_K) {
+        ph_gld<4, M>(p, h);
+        ph_gld<2, M>(p + 16 + 8 * g, h + 4);   // qh bytes 8 g ..
+    } else if constexpr (T == ST_Q6_K) {
+        ph_gld<1, !M>(p + 206, h);   // d in the high half
+    } else if constexpr (T == ST_IQ2_XS || T == ST_IQ3_XXS) {
+        ph_gld<1, M>(p, h);   // d in the low half
+    } else if constexpr (T == ST_IQ4_XS) {
+        ph_gld<2, M>(p, h);   // d, scales_h; scales_l
+    }
+}
+// What it decodes of half hb (columns 128 hb .. + 127). K step s (0..3) of
+// the half takes columns 32 s + 8 g .. + 7 of it, except IQ2_XS and
+// IQ3_XXS, whose lane group takes 32 g + 8 s .. + 7 (a lane's codes are then
+// adjacent bytes, ph_chunked).
+template <int T, bool M>
+__device__ __forceinline__ void ph_load_half(const uint8_t *p, int hb, int g, uint32_t *q) {
+    if constexpr (T == ST_Q2_K) {
+        ph_gld<2, M>(p + 16 + 32 * hb + 8 * g, q);
+        ph_gld<2, M>(p + 8 * hb, q + 2);   // its scale bytes
+    } else if constexpr (T == ST_Q3_K) {
+        ph_gld<2, M>(p + 32 + 32 * hb + 8 * g, q);
+    } else if constexpr (T == ST_Q4_K || T == ST_Q5_K) {
+        const int o = (T == ST_Q4_K ? 16 : 48) + 64 * hb + 8 * g;
+        ph_gld<2, M>(p + o, q);
+        ph_gld<2, M>(p + o + 32, q + 2);
+    } else if constexpr (T == ST_Q6_K) {
+        ph_gld<2, M>(p + 64 * hb + 8 * g, q);
+        ph_gld<2, M>(p + 64 * hb + 32 + 8 * g, q + 2);
+        ph_gld<2, M>(p + 128 + 32 * hb + 8 * g, q + 4);   // qh
+        ph_gld<2, M>(p + 192 + 8 * hb, q + 6);            // its scales
+    } else if constexpr (T == ST_IQ2_XS) {
+        ph_gld<2, !M>(p + 2 + 32 * hb + 8 * g, q);
+        ph_gld<1, !M>(p + 66 + 4 * hb, q + 2);   // the half's scales, byte g the lane group's
+    } else if constexpr (T == ST_IQ3_XXS) {
+        ph_gld<2, !M>(p + 2 + 32 * hb + 8 * g, q);
+        ph_gld<1, !M>(p + 66 + 16 * hb + 4 * g, q + 2);
+    } else if constexpr (T == ST_IQ4_XS) {
+#pragma unroll
+        for (int s = 0; s < 4; s++) ph_gld<2, M>(p + 8 + 16 * (4 * hb + s) + 8 * (g & 1), q + 2 * s);
+    } else {   // Q8_0: step 4 hb + s at 34 (4 hb + s), a dword for even s
+        ph_gld<2, !M>(p + 136 * hb + 2 + 8 * g, q);
+        ph_gld<1, M>(p + 136 * hb, q + 2);   // d in the low half
+        ph_gld<2, M>(p + 136 * hb + 36 + 8 * g, q + 3);
+        ph_gld<1, !M>(p + 136 * hb + 34, q + 5);
+        ph_gld<2, !M>(p + 136 * hb + 70 + 8 * g, q + 6);
+        ph_gld<1, M>(p + 136 * hb + 68, q + 8);
+        ph_gld<2, M>(p + 136 * hb + 104 + 8 * g, q + 9);
+        ph_gld<1, !M>(p + 136 * hb + 102, q + 11);
+    }
+}
+template <int T>
+__device__ __forceinline__ constexpr bool ph_chunked() { return T == ST_IQ2_XS || T == ST_IQ3_XXS; }
+
+__device__ __forceinline__ float ph_hlo(uint32_t v) { return f16_bits_to_f32(v & 0xFFFFu); }
+__device__ __forceinline__ float ph_hhi(uint32_t v) { return f16_bits_to_f32(v >> 16); }
+// Byte i of the dwords at h.
+__device__ __forceinline__ uint32_t ph_byte(const uint32_t *h, int i) { return (h[i >> 2] >> (8 * (i & 3))) & 255u; }
+// The 6-bit scale of sub-block j of Q4_K and Q5_K from the block's first 16
+// bytes (the packing of get_scale_min_k4, src/quants.c:96-102; scale byte i
+// is byte 4 + i).
+__device__ __forceinline__ uint32_t ph_scale_6(const uint32_t *h, int j) {
+    return j < 4 ? ph_byte(h, 4 + j) & 63u : (ph_byte(h, 8 + j) & 15u) | ((ph_byte(h, j) >> 6) << 4);
+}
+
+// What a lane decodes for a K step: the 8 codes (two operands for Q6_K) and,
+// for the STEP formats, the step's scale.
 struct PhB {
     ph_h8 b, b2;
     float sc;
 };
+// The IQ formats' table entries of K step s: grid and sign bytes, read a step
+// ahead of ph_decode.
+struct PhG {
+    uint2 gr, sg;
+};
 template <int T>
-__device__ __forceinline__ PhB ph_decode(const uint8_t *blk, const uint8_t *tab, const uint8_t *signs, int s, int g) {
-    PhB r;
-    if constexpr (T == ST_IQ2_XS) {
-        // qs u16 [4 s + g] at 2: grid index (9 bits), sign index (7 bits);
-        // 4-bit scale: nibble g >> 1 of byte 66 + s
-        const uint32_t v = ph_u16(blk + 2 + 2 * (4 * s + g));
-        const uint32_t sc = 2u * ((ph_u8(blk + 66 + s) >> (4 * (g >> 1))) & 15u) + 1u;
-        const uint2 gr = *(const __attribute__((address_space(3))) uint2 *)(size_t)pf_lds(tab + 8 * (v & 511u));
-        const uint2 sg = *(const __attribute__((address_space(3))) uint2 *)(size_t)pf_lds(signs + 8 * (v >> 9));
-        r.b = ph_codes_iq(gr, sg, ph_splat_u(sc << 10));
-    } else if constexpr (T == ST_IQ3_XXS) {
-        // qs bytes 8 s + 2 g, + 1 at 2 (grid indices, 4 bytes each); aux32 of
-        // step s at 66 + 4 s: sign index g at bit 7 g, 4-bit scale at 28
-        const uint32_t aux = ph_u32(blk + 66 + 4 * s);
-        const uint32_t ix = ph_u16(blk + 2 + 8 * s + 2 * g);
-        const uint32_t sc = 2u * (aux >> 28) + 1u;
-        uint2 gr;
-        gr.x = *(const __attribute__((address_space(3))) uint32_t *)(size_t)pf_lds(tab + 4 * (ix & 255u));
-        gr.y = *(const __attribute__((address_space(3))) uint32_t *)(size_t)pf_lds(tab + 4 * (ix >> 8));
-        const uint2 sg =
-            *(const __attribute__((address_space(3))) uint2 *)(size_t)pf_lds(signs + 8 * ((aux >> (7 * g)) & 127u));
-        r.b = ph_codes_iq(gr, sg, ph_splat_u(sc << 10));
-    } else if constexpr (T == ST_IQ4_XS) {
-        // qs[16 s + 8 (g & 1) + i] at 8, nibble g >> 1; 6-bit scale ls
-        const uint2 q = ph_u64(blk + 8 + 16 * s + 8 * (g & 1));
-        const uint32_t sh = 4u * (uint32_t)(g >> 1);
-        const uint2 lv = make_uint2(ph_iq4_levels(q.x >> sh), ph_iq4_levels(q.y >> sh));
-        r.b = ph_codes_sub(lv, ph_splat(1152.0f));
-        const uint32_t ls = ((ph_u8(blk + 4 + (s >> 1)) >> (4 * (s & 1))) & 15u) |
-                            (((ph_u16(blk + 2) >> (2 * s)) & 3u) << 4);
-        r.sc = ph_h2f(blk) * (float)((int32_t)ls - 32);
-    } else if constexpr (T == ST_Q5_K) {
-        // step s: 64-weight chunk j = s >> 1, nibble s & 1 of qs[32 j + l]
-        // (at 48) and bit s of qh[l] (at 16), l = 8 g .. 8 g + 7; 6-bit
-        // scale of sub-block s
-        const uint2 q = ph_u64(blk + 48 + 32 * (s >> 1) + 8 * g), h = ph_u64(blk + 16 + 8 * g);
-        const uint32_t nsh = 4u * (uint32_t)(s & 1);
-        const uint32_t c0 = ((q.x >> nsh) & 0x0F0F0F0Fu) | (((h.x >> s) & 0x01010101u) << 4);
-        const uint32_t c1 = ((q.y >> nsh) & 0x0F0F0F0Fu) | (((h.y >> s) & 0x01010101u) << 4);
-        const uint32_t sc = k_scale_6(blk + 4, s);
-        r.b = ph_codes_sub(make_uint2(c0, c1), ph_splat(1024.0f)) * (_Float16)(uint16_t)sc;
-    } else if constexpr (T == ST_Q6_K) {
-        // 128-half n6 = s >> 2, quarter qq = s & 3: low 4 bits from
-        // ql[64 n6 + 32 (qq & 1) + l] (nibble qq >> 1), high 2 bits from
-        // qh[32 n6 + l] bits 2 qq (at 128), l = 8 g .. 8 g + 7; int8 scale
-        // sc[8 n6 + 2 qq + (g >> 1)] (at 192) split as 16 a + b
-        const int n6 = s >> 2, qq = s & 3;
-        const uint2 q = ph_u64(blk + 64 * n6 + 32 * (qq & 1) + 8 * g), h = ph_u64(blk + 128 + 32 * n6 + 8 * g);
-        const uint32_t nsh = 4u * (uint32_t)(qq >> 1), hsh = 2u * (uint32_t)qq;
-        const uint32_t c0 = ((q.x >> nsh) & 0x0F0F0F0Fu) | (((h.x >> hsh) & 0x03030303u) << 4);
-        const uint32_t c1 = ((q.y >> nsh) & 0x0F0F0F0Fu) | (((h.y >> hsh) & 0x03030303u) << 4);
-        const int32_t sc = (int32_t)(int8_t)ph_u8(blk + 192 + 8 * n6 + 2 * qq + (g >> 1));
-        const ph_h8 q32 = ph_codes_sub(make_uint2(c0, c1), ph_splat(1056.0f));   // q - 32
-        r.b = q32 * (_Float16)(int16_t)(sc & 15);                               // (q - 32) b
-        r.b2 = q32 * (_Float16)(int16_t)(sc >> 4);                              // (q - 32) a
-    } else {   // Q8_0: block s (34 bytes at 34 s): d, then int8 qs
-        const uint2 q = ph_u64(blk + 34 * s + 2 + 8 * g);
-        r.b = ph_codes_sub(make_uint2(q.x ^ 0x80808080u, q.y ^ 0x80808080u), ph_splat(1152.0f));
-        r.sc = ph_h2f(blk + 34 * s);
+__device__ __forceinline__ PhG ph_gather(const uint32_t *q, const uint8_t *tab, const uint8_t *signs, int s) {
+    PhG r;
+    if constexpr (T == ST_IQ2_XS) {   // u16 s: grid index (9 bits), sign index (7 bits)
+        const uint32_t v = q[s >> 1] >> (16 * (s & 1));
+        r.gr = *(const __attribute__((address_space(3))) uint2 *)(size_t)pf_lds(tab + 8 * (v & 511u));
+        r.sg = *(const __attribute__((address_space(3))) uint2 *)(size_t)pf_lds(signs + 8 * ((v >> 9) & 127u));
+    } else if constexpr (T == ST_IQ3_XXS) {   // bytes 2 s, 2 s + 1: grid indices (4 codes each); sign index s at bit 7 s
+        const uint32_t ix = q[s >> 1] >> (16 * (s & 1));
+        r.gr.x = *(const __attribute__((address_space(3))) uint32_t *)(size_t)pf_lds(tab + 4 * (ix & 255u));
+        r.gr.y = *(const __attribute__((address_space(3))) uint32_t *)(size_t)pf_lds(tab + 4 * ((ix >> 8) & 255u));
+        r.sg = *(const __attribute__((address_space(3))) uint2 *)(size_t)pf_lds(signs + 8 * ((q[2] >> (7 * s)) & 127u));
     }
     return r;
 }
+template <int T>
+__device__ __forceinline__ PhB ph_decode(const uint32_t *h, const uint32_t *q, const PhG &G, int hb, int s, int g) {
+    PhB r;
+    if constexpr (T == ST_IQ2_XS) {   // 4-bit scale: nibble s >> 1 of the lane group's byte
+        r.b = ph_codes_iq(G.gr, G.sg, ph_splat_u((2u * ((q[2] >> (8 * g + 4 * (s >> 1))) & 15u) + 1u) << 10));
+    } else if constexpr (T == ST_IQ3_XXS) {   // 4-bit scale at bit 28
+        r.b = ph_codes_iq(G.gr, G.sg, ph_splat_u((2u * (q[2] >> 28) + 1u) << 10));
+    } else if constexpr (T == ST_IQ4_XS) {
+        // 8 bytes of the step's 16, nibble g >> 1; 6-bit scale ls of group 4 hb + s
+        const int j = 4 * hb + s;
+        const uint32_t sh = 4u * (uint32_t)(g >> 1);
+        const uint2 lv = make_uint2(ph_iq4_levels(q[2 * s] >> sh), ph_iq4_levels(q[2 * s + 1] >> sh));
+        r.b = ph_codes_sub(lv, ph_splat(1152.0f));
+        const uint32_t ls = ((h[1] >> (4 * j)) & 15u) | (((h[0] >> (16 + 2 * j)) & 3u) << 4);
+        r.sc = ph_hlo(h[0]) * (float)((int32_t)ls - 32);
+    } else if constexpr (T == ST_Q4_K || T == ST_Q5_K) {
+        // nibble s & 1 of bytes 32 (s >> 1) + 8 g .. (q[2 (s >> 1)], + 1); Q5_K: bit 4 hb + s of qh
+        const int j = 4 * hb + s, k = 2 * (s >> 1);
+        const uint32_t nsh = 4u * (uint32_t)(s & 1);
+        uint32_t c0 = (q[k] >> nsh) & 0x0F0F0F0Fu, c1 = (q[k + 1] >> nsh) & 0x0F0F0F0Fu;
+        if constexpr (T == ST_Q5_K) {
+            c0 |= ((h[4] >> j) & 0x01010101u) << 4;
+            c1 |= ((h[5] >> j) & 0x01010101u) << 4;
+        }
+        r.b = ph_codes_sub(make_uint2(c0, c1), ph_splat(1024.0f)) * (_Float16)(uint16_t)ph_scale_6(h, j);
+    } else if constexpr (T == ST_Q2_K) {
+        // bit pair s of the bytes; scale byte 2 s + (g >> 1) of the half, low nibble
+        const uint32_t c0 = (q[0] >> (2 * s)) & 0x03030303u, c1 = (q[1] >> (2 * s)) & 0x03030303u;
+        const uint32_t sc = (q[2 + (s >> 1)] >> (16 * (s & 1) + 8 * (g >> 1))) & 15u;
+        r.b = ph_codes_sub(make_uint2(c0, c1), ph_splat(1024.0f)) * (_Float16)(uint16_t)sc;
+    } else if constexpr (T == ST_Q3_K) {
+        // bit pair s of the bytes, high bit 4 hb + s of hmask; scale j = 8 hb + 2 s + (g >> 1): nibble hb of
+        // byte 2 s + (g >> 1), its high bits 2 (j >> 2) of byte 8 + (j & 3)
+        const int b = 4 * hb + s;
+        const uint32_t c0 = ((q[0] >> (2 * s)) & 0x03030303u) | (((h[0] >> b) & 0x01010101u) << 2);
+        const uint32_t c1 = ((q[1] >> (2 * s)) & 0x03030303u) | (((h[1] >> b) & 0x01010101u) << 2);
+        const uint32_t gs = 8u * (uint32_t)(g >> 1);
+        const uint32_t lo = (h[2 + (s >> 1)] >> (16 * (s & 1) + 4 * hb + gs)) & 15u;
+        const uint32_t hi = (h[4] >> (16 * (s & 1) + 2 * (2 * hb + (s >> 1)) + gs)) & 3u;
+        r.b = ph_codes_sub(make_uint2(c0, c1), ph_splat(1028.0f)) * (_Float16)(int16_t)((int32_t)(lo | (hi << 4)) - 32);
+    } else if constexpr (T == ST_Q6_K) {
+        // quarter s: low 4 bits from ql[32 (s & 1) + 8 g ..] (nibble s >> 1), high 2 from qh bits 2 s; int8 scale
+        // 2 s + (g >> 1) of the half, split as 16 a + b
+        const int k = 2 * (s & 1);
+        const uint32_t nsh = 4u * (uint32_t)(s >> 1), hsh = 2u * (uint32_t)s;
+        const uint32_t c0 = ((q[k] >> nsh) & 0x0F0F0F0Fu) | (((q[4] >> hsh) & 0x03030303u) << 4);
+        const uint32_t c1 = ((q[k + 1] >> nsh) & 0x0F0F0F0Fu) | (((q[5] >> hsh) & 0x03030303u) << 4);
+        const int32_t sc = (int32_t)(int8_t)((q[6 + (s >> 1)] >> (16 * (s & 1) + 8 * (g >> 1))) & 255u);
+        const ph_h8 q32 = ph_codes_sub(make_uint2(c0, c1), ph_splat(1056.0f));   // q - 32
+        r.b = q32 * (_Float16)(int16_t)(sc & 15);                               // (q - 32) b
+        r.b2 = q32 * (_Float16)(int16_t)(sc >> 4);                              // (q - 32) a
+    } else {   // Q8_0
+        r.b = ph_codes_sub(make_uint2(q[3 * s] ^ 0x80808080u, q[3 * s + 1] ^ 0x80808080u), ph_splat(1152.0f));
+        r.sc = ph_hlo(q[3 * s + 2]);
+    }
+    return r;
+}
+// The mins of a half as a matrix operand against the record's sum groups:
+// lane group g has columns 32 g .. + 31, three terms of each 16-column sum.
+template <int T>
+__device__ __forceinline__ ph_h8 ph_mins(const uint32_t *h, const uint32_t *q, int hb, int g) {
+    _Float16 a, b;
+    const uint32_t gs = 8u * (uint32_t)g;
+    if constexpr (T == ST_Q2_K) {
+        const uint32_t v = q[2 + (g >> 1)] >> (16 * (g & 1));   // scale bytes 2 g, 2 g + 1 of the half: high nibbles
+        a = (_Float16)(uint16_t)((v >> 4) & 15u);
+        b = (_Float16)(uint16_t)((v >> 12) & 15u);
+    } else {
+        const uint32_t m = hb == 0 ? (h[2] >> gs) & 63u : ((h[3] >> (gs + 4)) & 15u) | (((h[2] >> (gs + 6)) & 3u) << 4);
+        a = b = (_Float16)(uint16_t)m;
+    }
+    return ph_h8{a, a, a, b, b, b, (_Float16)0.0f, (_Float16)0.0f};
+}
 
 // ----------------------------------------------------------- projection --
-// One projection workgroup (see the top of the file). GU: rows r0 .. r0 +
-// R / 2 - 1 of gate (W0) and up (W1), h[pair][row] = silu(gate) * up in
-// f32; down: rows r0 .. r0 + R - 1 of W0, out[pair][row] in f32. Stepping
-// wave w (w < R / RW, RW = 16 NT) computes RW rows (NT N tiles) x the
-// unit's one or two 16-pair M tiles (GU: waves w and w + R / (2 RW) the
-// same rows of gate and up); the other waves stage records only.
+template <bool B> struct PhBool { static constexpr bool value = B; };
+
+// One projection workgroup (see the top of the file). GU: wave w computes
+// rows r0 + 16 w .. of gate (W0, tile 0) and up (W1, tile 1), h[pair][row] =
+// silu(gate) * up in f32; down: rows r0 + 32 w .. of W0, out[pair][row] in
+// f32. rows: those of the matrix; a wave past them only stages records.
 template <int T, bool GU, int MT>
 __device__ __forceinline__ void ph_proj(uint8_t *smem, const uint8_t *W0, const uint8_t *W1, uint64_t row_bytes,
-                                        int64_t nb, const uint8_t *rec, const uint32_t *roff, const int32_t *pair,
-                                        const float *srow, int nv, int64_t r0, float *__restrict__ out,
+                                        int64_t nb, const uint8_t *rec, const int64_t *roff, const int32_t *pair,
+                                        const float *srow, int nv, int64_t r0, int64_t rows, float *__restrict__ out,
                                         int64_t ld_out) {
-    constexpr int BB = PhFmt<T>::BB, PW = PhFmt<T>::PW, SW = PhFmt<T>::SW, R = PhFmt<T>::R;
-    constexpr int NT = PhFmt<T>::NT, RW = 16 * NT, AW = R / RW, HALF = AW / 2;
-    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), l = threadIdx.x & 63, n = l & 15,
-              g = l >> 4;
-    const bool on = w < AW;
-    const uint8_t *Wm = (GU && w >= HALF) ? W1 : W0;
-    const int64_t grow = r0 + RW * (GU ? w % HALF : w);   // the wave's first global row
-    auto a_stage = [&](int b) { return smem + (uint32_t)(b & 1) * PH_ABYTES; };
-    auto w_stage = [&](int b) { return smem + 2 * PH_ABYTES + (uint32_t)b % SW * PhLds<T>::W; };
-    const uint8_t *tab = smem + PhLds<T>::TAB, *signs = smem + PhLds<T>::SIGNS;
-    ph_fill_tables<T>(smem);   // published by the first block's barrier
-    PhDma<T, GU> dma;
-    dma.init(roff, row_bytes, r0, nv);
-    pf_f32x4 acc[NT][2];
+    typedef PhFmt<T> F;
+    constexpr int NT = 2, G = MT <= 2 ? F::G : F::GL, QN = F::QN, HN = F::HN, HT = GU ? 1 : 2;
+    // a group's bytes of a row, from the dword at or below its start (odd
+    // blocks of a format of 4 k + 2 bytes start 2 bytes past one; only G = 1
+    // groups do), as PW pieces; KW wave instructions a tile
+    constexpr int PW = (G * F::BB + (G == 1 && F::BB % 4 ? 2 : 0) + 15) / 16, KW = (16 * PW + 63) / 64;
+    constexpr uint32_t O_W = 2u * 16u * MT * PH_LREC;
+    static_assert(O_W + PH_WAVES * NT * 16 * 16 * PW <= (T == ST_IQ2_XS || T == ST_IQ3_XXS ? PH_O_TAB : PH_O_ROWS), "LDS");
+    const int tid = (int)threadIdx.x, l = tid & 63, n = l & 15, g = l >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t grow = r0 + 16 * HT * w;   // the wave's first row
+    const bool on = grow < rows;
+    const int nbi = (int)nb, nst = 2 * nbi;
+    const uint8_t *tab = smem + PH_O_TAB, *signs = smem + PH_O_SIGNS;
+    ph_fill_tables<T>(smem);   // published by the first barrier
+    // records: piece tid + 512 i of a half is row m = piece / 32 of the unit,
+    // 16-byte column group piece % 32 (hi, then lo); a K step's four lane
+    // groups read adjacent pieces
+    const uint8_t *asrc[MT];
+    uint32_t adst[MT];
+    const uint8_t *ssrc = nullptr;
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+        const int p = tid + 512 * i, m = p >> 5, c = p & 31, cg = c & 15;
+        asrc[i] = rec + roff[m] + 16 * c;
+        adst[i] = (uint32_t)(m * PH_LREC + 256 * (c >> 4) + 16 * (ph_chunked<T>() ? 4 * (cg & 3) + (cg >> 2) : cg));
+    }
+    if (F::MIN) ssrc = rec + roff[tid < 64 * MT ? tid >> 2 : 0] + 512 + 16 * (tid & 3);
+    // Loads return in order, so the records of units of up to two M tiles are
+    // fetched AD halves ahead: a wait for records issued after a weight group
+    // is one for that group too.
+    constexpr int AD = MT <= 2 ? 4 : 1;   // divides a turn's halves
+    ph_u4 ar[AD][MT], sr[AD];
+    auto a_load = [&](int t, int slot) {
+        t = t < nst ? t : nst - 1;
+#pragma unroll
+        for (int i = 0; i < MT; i++) ar[slot][i] = *(const ph_u4 *)(asrc[i] + (uint32_t)t * PH_REC);
+        if (F::MIN) sr[slot] = *(const ph_u4 *)(ssrc + (uint32_t)t * PH_REC);
+    };
+    auto a_store = [&](int t, int slot) {
+        uint8_t *st = smem + (uint32_t)(t & 1) * (16 * MT * PH_LREC);
+#pragma unroll
+        for (int i = 0; i < MT; i++) *(ph_u4 *)(st + adst[i]) = ar[slot][i];
+        if (F::MIN && tid < 64 * MT) *(ph_u4 *)(st + (tid >> 2) * PH_LREC + 512 + 16 * (tid & 3)) = sr[slot];
+    };
+    // weights: piece q = 64 k + lane of a tile's group is row q / PW, bytes
+    // 16 (q % PW) .. of it; pieces past the row's last block take the group's
+    // first (the last one that holds block bytes may run up to 14 bytes past
+    // the matrix, into the 256 that every device buffer of the library
+    // carries past its data, dev_bytes in sepia_hip.c)
+    uint32_t wrow[KW], wcol[KW];
+#pragma unroll
+    for (int k = 0; k < KW; k++) {
+        const int q = 64 * k + l < 16 * PW ? 64 * k + l : 0, m = q / PW;
+        wrow[k] = on ? (uint32_t)((uint64_t)(grow + m) * row_bytes) : 0u;
+        wcol[k] = 16u * (uint32_t)(q - m * PW);
+    }
+    const uint8_t *Wt[NT] = {W0, GU ? W1 : W0 + (on ? 16 * row_bytes : 0)};
+    uint8_t *wl = smem + O_W + (uint32_t)w * (NT * 16 * 16 * PW);
+    ph_u4 wr[NT][KW];
+    auto w_load = [&](int b) {   // the group of blocks b ..
+        const uint32_t at = ((uint32_t)b * F::BB) & ~3u, left = (uint32_t)nbi * F::BB - at;
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int k = 0; k < KW; k++) {
+                typedef ph_u4 U4 __attribute__((aligned(4)));
+                wr[t][k] = *(const U4 *)(Wt[t] + at + (uint64_t)(wrow[k] + (wcol[k] < left ? wcol[k] : 0u)));
+            }
+    };
+    auto w_store = [&]() {
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int k = 0; k < KW; k++)
+                if (64 * (k + 1) <= 16 * PW || 64 * k + l < 16 * PW)
+                    *(ph_u4 *)(wl + t * (16 * 16 * PW) + 1024 * k + 16 * l) = wr[t][k];
+    };
+    pf_f32x4 acc[NT][MT], cb[NT][MT], cb2[T == ST_Q6_K ? NT : 1][T == ST_Q6_K ? MT : 1],
+        cm[F::MIN ? NT : 1][F::MIN ? MT : 1];
+    const pf_f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int t = 0; t < NT; t++)
 #pragma unroll
-        for (int mt = 0; mt < 2; mt++) acc[t][mt] = pf_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const int nbi = (int)nb;
-    dma.issue_a(0, a_stage(0), rec);
-    for (int c = 0; c < SW - 1 && c < nbi; c++) dma.issue_w(c, w_stage(c), Wm);
-    constexpr int APB = 16 * PH_AP;   // bytes of a staged record
-    constexpr int KW = PhDma<T, GU>::KW;
-    for (int b = 0; b < nbi; b++) {
-        // everything up to A_b and W_b; the weights of blocks b + 1 .. b + SW - 2 may fly
-        const int ahead = (nbi - 1 - b) < (SW - 2) ? (nbi - 1 - b) : (SW - 2);
-        pq_wait_vm<KW * (SW - 2)>((on ? KW : 0) * ahead);
-        // the blocks at offset o of their staged rows (rows of 4-byte multiples)
-        const uint8_t *blk[NT];
+        for (int mt = 0; mt < MT; mt++) acc[t][mt] = zero;
+    // half hb of block b (o: where it starts in the staged group)
+    auto half = [&](auto mis, int o, int hb) {
+        constexpr bool M = decltype(mis)::value;
+        const uint8_t *As = smem + (uint32_t)hb * (16 * MT * PH_LREC) + n * PH_LREC + 16 * g;
+        uint32_t q[NT][QN], h[NT][HN];
 #pragma unroll
-        for (int t = 0; t < NT; t++)
-            blk[t] = w_stage(b) + (uint32_t)(RW * w + 16 * t + n) * (PW * 16) + (((uint32_t)b * BB) & 3u);
-        asm volatile("" ::: "memory");
-        __syncthreads();   // every wave's record pieces of A_b, the tables
-        asm volatile("" ::: "memory");
-        if (b + 1 < nbi) dma.issue_a(b + 1, a_stage(b + 1), rec);
-        if (b + SW - 1 < nbi) dma.issue_w(b + SW - 1, w_stage(b + SW - 1), Wm);
-        if (!on) continue;
-        const uint8_t *As = a_stage(b);
-        pf_f32x4 cb[NT][2], cb2[NT][2];
-#pragma unroll
-        for (int t = 0; t < NT; t++)
-#pragma unroll
-            for (int mt = 0; mt < 2; mt++) {
-                cb[t][mt] = pf_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                cb2[t][mt] = pf_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            }
-        // Software-pipelined by one K step: step s + 1's codes (LDS
-        // gathers and their VALU) and activation planes are read before
-        // step s's matrix ops are issued (the scheduling barrier keeps that
-        // order), so the gathers' latency runs under the MFMAs.
-        PhB B[NT];
-#pragma unroll
-        for (int t = 0; t < NT; t++) B[t] = ph_decode<T>(blk[t], tab, signs, 0, g);
-        ph_h8 ah[MT], al[MT];
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            const uint8_t *ap = As + (16 * mt + n) * APB + 16 * g;
-            ah[mt] = *(const __attribute__((address_space(3))) ph_h8 *)(size_t)pf_lds(ap);
-            al[mt] = *(const __attribute__((address_space(3))) ph_h8 *)(size_t)pf_lds(ap + 512);
+        for (int t = 0; t < NT; t++) {
+            const uint8_t *blk = wl + (16 * t + n) * (16 * PW) + o;
+            ph_load_half<T, M>(blk, hb, g, q[t]);
+            ph_load_head<T, M>(blk, g, h[t]);
         }
+        if (hb == 0) {
 #pragma unroll
-        for (int s = 0; s < 8; s++) {
-            PhB Bn[NT];
-            ph_h8 ahn[MT], aln[MT];
-            if (s + 1 < 8) {
-#pragma unroll
-                for (int t = 0; t < NT; t++) Bn[t] = ph_decode<T>(blk[t], tab, signs, s + 1, g);
+            for (int t = 0; t < NT; t++)
 #pragma unroll
                 for (int mt = 0; mt < MT; mt++) {
-                    const uint8_t *ap = As + (16 * mt + n) * APB + 64 * (s + 1) + 16 * g;
-                    ahn[mt] = *(const __attribute__((address_space(3))) ph_h8 *)(size_t)pf_lds(ap);
-                    aln[mt] = *(const __attribute__((address_space(3))) ph_h8 *)(size_t)pf_lds(ap + 512);
+                    cb[t][mt] = zero;
+                    if constexpr (T == ST_Q6_K) cb2[t][mt] = zero;
+                    if constexpr (F::MIN) cm[t][mt] = zero;
                 }
+        }
+        // Pipelined by one K step: step s + 1's table entries and activations
+        // are on their way from LDS while step s's matrix ops run; its codes
+        // are made of them after.
+        PhB B[NT];
+        PhG Gt[NT];
+        ph_h8 a1[2];
+#pragma unroll
+        for (int t = 0; t < NT; t++) Gt[t] = ph_gather<T>(q[t], tab, signs, 0);
+        auto a_read = [&](int s, int mt, int pl) {
+            return *(const __attribute__((address_space(3))) ph_h8 *)(size_t)pf_lds(As + 16 * mt * PH_LREC + 256 * pl + 64 * s);
+        };
+#pragma unroll
+        for (int pl = 0; pl < 2; pl++) a1[pl] = a_read(0, 0, pl);
+#pragma unroll
+        for (int t = 0; t < NT; t++) B[t] = ph_decode<T>(h[t], q[t], Gt[t], hb, 0, g);
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            ph_h8 a2[2][2];
+            a2[0][0] = a1[0];
+            a2[0][1] = a1[1];
+            if (s + 1 < 4) {
+#pragma unroll
+                for (int t = 0; t < NT; t++) Gt[t] = ph_gather<T>(q[t], tab, signs, s + 1);
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) {
+                if (mt + 1 < MT) {
+#pragma unroll
+                    for (int pl = 0; pl < 2; pl++) a2[(mt + 1) & 1][pl] = a_read(s, mt + 1, pl);
+                } else if (s + 1 < 4) {
+#pragma unroll
+                    for (int pl = 0; pl < 2; pl++) a1[pl] = a_read(s + 1, 0, pl);
+                }
+                const ph_h8 ah = a2[mt & 1][0], al = a2[mt & 1][1];
 #pragma unroll
                 for (int t = 0; t < NT; t++) {
-                    if constexpr (PhFmt<T>::STEP) {
-                        pf_f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[mt], B[t].b, pf_f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-                        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[mt], B[t].b, c, 0, 0, 0);
+                    if constexpr (F::STEP) {
+                        pf_f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, B[t].b, zero, 0, 0, 0);
+                        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, B[t].b, c, 0, 0, 0);
 #pragma unroll
-                        for (int i = 0; i < 4; i++) acc[t][mt][i] = __builtin_fmaf(B[t].sc, c[i], acc[t][mt][i]);
+                        for (int k = 0; k < 4; k++) acc[t][mt][k] = __builtin_fmaf(B[t].sc, c[k], acc[t][mt][k]);
                     } else {
-                        cb[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[mt], B[t].b, cb[t][mt], 0, 0, 0);
-                        cb[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[mt], B[t].b, cb[t][mt], 0, 0, 0);
+                        cb[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, B[t].b, cb[t][mt], 0, 0, 0);
+                        cb[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, B[t].b, cb[t][mt], 0, 0, 0);
                         if constexpr (T == ST_Q6_K) {
-                            cb2[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[mt], B[t].b2, cb2[t][mt], 0, 0, 0);
-                            cb2[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[mt], B[t].b2, cb2[t][mt], 0, 0, 0);
+                            cb2[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, B[t].b2, cb2[t][mt], 0, 0, 0);
+                            cb2[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, B[t].b2, cb2[t][mt], 0, 0, 0);
                         }
                     }
                 }
             }
-            if (s + 1 < 8) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (s + 1 < 4) {
 #pragma unroll
-                for (int t = 0; t < NT; t++) B[t] = Bn[t];
+                for (int t = 0; t < NT; t++) B[t] = ph_decode<T>(h[t], q[t], Gt[t], hb, s + 1, g);
+            }
+        }
+        if constexpr (F::MIN) {   // mins . sums
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                const ph_h8 mb = ph_mins<T>(h[t], q[t], hb, g);
 #pragma unroll
                 for (int mt = 0; mt < MT; mt++) {
-                    ah[mt] = ahn[mt];
-                    al[mt] = aln[mt];
+                    const ph_h8 sa =
+                        *(const __attribute__((address_space(3))) ph_h8 *)(size_t)pf_lds(As + 16 * mt * PH_LREC + 512);
+                    cm[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(sa, mb, cm[t][mt], 0, 0, 0);
                 }
             }
         }
+        if (!F::STEP && hb == 1) {
 #pragma unroll
-        for (int t = 0; t < NT; t++) {
-            if constexpr (T == ST_IQ2_XS || T == ST_IQ3_XXS) {
-                const float d = ph_h2f(blk[t]) * (T == ST_IQ2_XS ? 2048.0f : 4096.0f);   // 2^14 / 8, 2^14 / 4
+            for (int t = 0; t < NT; t++) {
+                // IQ: 2^14 / 8, 2^14 / 4
+                const float d = T == ST_IQ2_XS    ? ph_hlo(h[t][0]) * 2048.0f
+                                : T == ST_IQ3_XXS ? ph_hlo(h[t][0]) * 4096.0f
+                                : T == ST_Q3_K    ? ph_hhi(h[t][HN - 1])
+                                : T == ST_Q6_K    ? ph_hhi(h[t][0])
+                                                  : ph_hlo(h[t][0]);
 #pragma unroll
                 for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-                    for (int i = 0; i < 4; i++) acc[t][mt][i] = __builtin_fmaf(d, cb[t][mt][i], acc[t][mt][i]);
-            } else if constexpr (T == ST_Q6_K) {
-                const float d = ph_h2f(blk[t] + 208);
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++)
-                        acc[t][mt][i] =
-                            __builtin_fmaf(d, __builtin_fmaf(16.0f, cb2[t][mt][i], cb[t][mt][i]), acc[t][mt][i]);
-            } else if constexpr (T == ST_Q5_K) {   // d C - dmin sum_j m_j S_j, the min terms on the f32 matrix cores
-                const float d = ph_h2f(blk[t]), dmin = ph_h2f(blk[t] + 2);
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++) {
-                    pf_f32x4 cm = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                    for (int h = 0; h < 2; h++) {
-                        // A[pair][k] = S_(4 h + k) of pair 16 mt + n; B[k][row n] = m_(4 h + k)
-                        const float sa = *(const __attribute__((address_space(3))) float *)(size_t)pf_lds(
-                            As + (16 * mt + n) * APB + 1024 + 4 * (4 * h + g));
-                        const float mb = (float)k_min_6(blk[t] + 4, 4 * h + g);
-                        cm = __builtin_amdgcn_mfma_f32_16x16x4f32(sa, mb, cm, 0, 0, 0);
+                    for (int k = 0; k < 4; k++) {
+                        float c = cb[t][mt][k];
+                        if constexpr (T == ST_Q6_K) c = __builtin_fmaf(16.0f, cb2[t][mt][k], c);
+                        acc[t][mt][k] = __builtin_fmaf(d, c, acc[t][mt][k]);
+                        if constexpr (F::MIN)
+                            acc[t][mt][k] = __builtin_fmaf(-ph_hhi(h[t][0]), cm[t][mt][k], acc[t][mt][k]);
                     }
-#pragma unroll
-                    for (int i = 0; i < 4; i++)
-                        acc[t][mt][i] = __builtin_fmaf(-dmin, cm[i], __builtin_fmaf(d, cb[t][mt][i], acc[t][mt][i]));
-                }
             }
+        }
+    };
+    // Every load is unconditional (past the last block, the last one again;
+    // waves without rows, row 0): a wait after a branch around loads would be
+    // for all of them.
+#pragma unroll
+    for (int i = 0; i < AD; i++) a_load(i, i);
+    w_load(0);
+    a_store(0, 0);
+    if constexpr (AD > 1) a_load(AD, 0);
+    __syncthreads();
+    // a group, or two blocks, a turn: a block's alignment, a record slot's
+    // registers and where a group starts are then known at compile time
+    constexpr int U = G < 2 ? 2 : G;
+    for (int b0 = 0; b0 < nbi; b0 += U) {
+#pragma unroll
+        for (int i = 0; i < 2 * U; i++) {
+            const int b = b0 + i / 2, hb = i % 2, t_st = 2 * b + hb;
+            if (b >= nbi) break;
+            if constexpr (AD == 1) a_load(t_st + 1, 0);
+            if (i % (2 * G) == 0) {   // a new group
+                w_store();
+                w_load(b + G < nbi ? b + G : b);
+                asm volatile("" ::: "memory");
+            }
+            if (on) {
+                const int o = (i / 2 % G) * F::BB + (G == 1 && F::BB % 4 ? i / 2 * 2 : 0);
+                if (F::BB % 4 && (i / 2) % 2) half(PhBool<true>{}, o, hb);
+                else half(PhBool<false>{}, o, hb);
+            }
+            // the next half's records to LDS (the buffer the half before used)
+            if constexpr (AD == 1) {
+                a_store(t_st + 1, 0);
+            } else {
+                a_store(t_st + 1, (i + 1) % AD);
+                a_load(t_st + 1 + AD, (i + 1) % AD);
+            }
+            __syncthreads();
         }
     }
-    // y = s_pair * acc; lane: pairs 16 mt + 4 g + i, rows grow + 16 t + n
+    if (!on) return;
+    // y = s_pair * acc; lane: pairs 16 mt + 4 g + k, rows grow + 16 t + n
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float sp = srow[16 * mt + 4 * g + i];
-#pragma unroll
-            for (int t = 0; t < NT; t++) acc[t][mt][i] *= sp;
-        }
-    if constexpr (GU) {
-        __syncthreads();   // every wave is done with the stages
-        float *xch = (float *)smem + ((w % HALF) * 64 + l) * (8 * NT);
-        if (on && w >= HALF) {
-#pragma unroll
-            for (int t = 0; t < NT; t++)
-#pragma unroll
-                for (int mt = 0; mt < 2; mt++) *(pf_f32x4 *)(xch + 8 * t + 4 * mt) = acc[t][mt];
-        }
-        __syncthreads();
-        if (!on || w >= HALF) return;
-#pragma unroll
-        for (int t = 0; t < NT; t++)
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
-                const pf_f32x4 u = *(const pf_f32x4 *)(xch + 8 * t + 4 * mt);
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int m = 16 * mt + 4 * g + i;
-                    if (m < nv) out[(int64_t)pair[m] * ld_out + grow + 16 * t + n] = silu_f32(acc[t][mt][i]) * u[i];
-                }
+        for (int k = 0; k < 4; k++) {
+            const int m = 16 * mt + 4 * g + k;
+            if (m >= nv) continue;
+            const float sp = srow[m];
+            float *o = out + (int64_t)pair[m] * ld_out + grow + n;
+            if constexpr (GU) {
+                o[0] = silu_f32(acc[0][mt][k] * sp) * (acc[1][mt][k] * sp);
+            } else {
+                o[0] = acc[0][mt][k] * sp;
+                o[16] = acc[1][mt][k] * sp;
             }
-    } else {
-        if (!on) return;
-#pragma unroll
-        for (int t = 0; t < NT; t++)
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int m = 16 * mt + 4 * g + i;
-                    if (m < nv) out[(int64_t)pair[m] * ld_out + grow + 16 * t + n] = acc[t][mt][i];
-                }
-    }
+        }
 }
 
-// The launch has one workgroup per row slice (gate/up: 64 rows of each
-// matrix; down: 128 rows); a format with R = 256 rows covers two slices (see
-// ph_slice).
-#define PH_DISPATCH(TYPE, GU, R0, ...)                                                               \
-    do {                                                                                             \
-        switch (TYPE) {                                                                              \
-        case ST_IQ2_XS: PH_CALL(ST_IQ2_XS, GU, R0, __VA_ARGS__); break;                              \
-        case ST_IQ3_XXS: PH_CALL(ST_IQ3_XXS, GU, R0, __VA_ARGS__); break;                            \
-        case ST_IQ4_XS: PH_CALL(ST_IQ4_XS, GU, R0, __VA_ARGS__); break;                              \
-        case ST_Q5_K: PH_CALL(ST_Q5_K, GU, R0, __VA_ARGS__); break;                                  \
-        case ST_Q6_K: PH_CALL(ST_Q6_K, GU, R0, __VA_ARGS__); break;                                  \
-        case ST_Q8_0: PH_CALL(ST_Q8_0, GU, R0, __VA_ARGS__); break;                                  \
-        default: break;                                                                              \
-        }                                                                                            \
-    } while (0)
-#define PH_CALL(T, GU, R0, smem, W0, W1, row_bytes, nb, rec, roff, pair, srow, nv, out, ld_out)      \
-    do {                                                                                             \
-        if (nv > 16) ph_proj<T, GU, 2>(smem, W0, W1, row_bytes, nb, rec, roff, pair, srow, nv, R0, out, ld_out); \
-        else ph_proj<T, GU, 1>(smem, W0, W1, row_bytes, nb, rec, roff, pair, srow, nv, R0, out, ld_out);        \
-    } while (0)
-// Formats staged 128 rows at a time (the others 256).
-__device__ __forceinline__ bool ph_rows128(int32_t t) { return t == ST_Q6_K || t == ST_Q8_0; }
-// The first row slice of slot x, or -1 for none: formats staged 256
-// rows at a time take slices 2 x, 2 x + 1 in the slots x < gridDim.x / 2.
-// Keeping the active slots at consecutive x spreads them over all 8 XCDs
-// (the hardware deals consecutive workgroup ids to the XCDs in turn: with
-// rows of 48 workgroups, active even x alone would land on 4 of them).
-__device__ __forceinline__ int64_t ph_slice(int32_t t, int32_t x) {
-    if (ph_rows128(t)) return x;
-    return x < (int32_t)gridDim.x / 2 ? 2 * (int64_t)x : -1;
+// The unit's row tables: record offset, pair and scale of its rows (those
+// past its pairs repeat the first; their outputs are discarded).
+__device__ __forceinline__ void ph_unit_rows(const int32_t *pairs, int nv, bool by_token, int32_t n_sel, int64_t ldr,
+                                             const float *scale, uint8_t *smem, int64_t *&roff, int32_t *&pair,
+                                             float *&srow) {
+    roff = (int64_t *)(smem + PH_O_ROWS);
+    pair = (int32_t *)(roff + PH_UM);
+    srow = (float *)(pair + PH_UM);
+    if (threadIdx.x < PH_UM) {
+        const int32_t p = pairs[threadIdx.x < (unsigned)nv ? (int)threadIdx.x : 0];
+        const int64_t row = by_token ? (int64_t)(p / n_sel) : (int64_t)p;
+        pair[threadIdx.x] = p;
+        roff[threadIdx.x] = row * ldr;
+        srow[threadIdx.x] = scale[row];
+    }
+    __syncthreads();
+}
+
+// The launch has one workgroup per row slice (gate/up: 128 rows of each
+// matrix; down: 256 rows) and unit.
+#define PH_CASE(T, GU)                                                                                         \
+    case T:                                                                                                    \
+        if (nv > 48) ph_proj<T, GU, 4>(smem, W0, W1, row_bytes, nb, rec, roff, pair, srow, nv, r0, rows, out, ld_out); \
+        else if (nv > 32) ph_proj<T, GU, 3>(smem, W0, W1, row_bytes, nb, rec, roff, pair, srow, nv, r0, rows, out, ld_out); \
+        else if (nv > 16) ph_proj<T, GU, 2>(smem, W0, W1, row_bytes, nb, rec, roff, pair, srow, nv, r0, rows, out, ld_out); \
+        else ph_proj<T, GU, 1>(smem, W0, W1, row_bytes, nb, rec, roff, pair, srow, nv, r0, rows, out, ld_out); \
+        break;
+template <bool GU>
+__device__ __forceinline__ void ph_run(int32_t type, uint8_t *smem, const uint8_t *W0, const uint8_t *W1,
+                                       uint64_t row_bytes, int64_t nb, const uint8_t *rec, const int64_t *roff,
+                                       const int32_t *pair, const float *srow, int nv, int64_t r0, int64_t rows,
+                                       float *out, int64_t ld_out) {
+    switch (type) {
+        PH_CASE(ST_IQ2_XS, GU)
+        PH_CASE(ST_IQ3_XXS, GU)
+        PH_CASE(ST_IQ4_XS, GU)
+        PH_CASE(ST_Q2_K, GU)
+        PH_CASE(ST_Q3_K, GU)
+        PH_CASE(ST_Q4_K, GU)
+        PH_CASE(ST_Q5_K, GU)
+        PH_CASE(ST_Q6_K, GU)
+        PH_CASE(ST_Q8_0, GU)
+    default: break;
+    }
 }
 // 256-column blocks of a row (a projection's n_blocks counts Q8_0's
 // 32-column blocks; its 256-column block is eight of them, 272 bytes).
 __device__ __forceinline__ int64_t ph_nb(int32_t t, int64_t n_blocks) { return t == ST_Q8_0 ? n_blocks / 8 : n_blocks; }
 
-// Gate/up: workgroup (64-row slice bx of I, unit by); hf[p][row] = silu(gate
+// Gate/up: workgroup (128-row slice bx of I, unit by); hf[p][row] = silu(gate
 // . x_t) * (up . x_t) in f32 for the unit's pairs p (token t = p / n_sel).
 // The host launches it only when every projection of the layer has one of
 // the formats above, with 4-byte-aligned rows, and H and I are multiples of
@@ -621,48 +756,41 @@ extern "C" __global__ __launch_bounds__(64 * PH_WAVES) void sepia_ph_gateup(
     PfProj gate, PfProj up, PfProj s_gate, PfProj s_up, int32_t n_routed, int32_t n_sel, int64_t I, int64_t H,
     const uint8_t *__restrict__ phx, const float *__restrict__ phxs, const int32_t *__restrict__ list,
     const int32_t *__restrict__ units, const int32_t *__restrict__ n_units, float *__restrict__ hf) {
-    const PfSlot slot = pf_slot();
+    const PfSlot slot = pf_slot(n_units[0]);
     if (slot.y >= n_units[0]) return;
     extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
-    uint8_t *smem = pf_smem;
     const int32_t *un = units + 3 * slot.y;
     const int32_t e = un[0], nv = un[2];
     const bool routed = e < n_routed;
     const PfProj &G = routed ? gate : s_gate, &U = routed ? up : s_up;
     const int64_t ei = routed ? e : e - n_routed;
-    const uint8_t *wg = G.base + ei * G.stride, *wu = U.base + ei * U.stride;
-    const int64_t sl = ph_slice(G.type, slot.x);
-    if (sl < 0) return;
-    uint32_t *roff;
+    int64_t *roff;
     int32_t *pair;
     float *srow;
-    pq_unit_rows(list + un[1], nv, true, n_sel, (H / 256) * PH_REC, phxs, smem, roff, pair, srow);
-    PH_DISPATCH(G.type, true, sl * 64, smem, wg, wu, G.row_bytes, ph_nb(G.type, G.n_blocks), phx, roff,
-                pair, srow, nv, hf, I);
+    ph_unit_rows(list + un[1], nv, true, n_sel, (H / 128) * PH_REC, phxs, pf_smem, roff, pair, srow);
+    ph_run<true>(G.type, pf_smem, G.base + ei * G.stride, U.base + ei * U.stride, G.row_bytes, ph_nb(G.type, G.n_blocks),
+                 phx, roff, pair, srow, nv, slot.x * 128, I, hf, I);
 }
 
-// Down: workgroup (128-row slice bx of H, unit by); yp[p][row] = down_e .
+// Down: workgroup (256-row slice bx of H, unit by); yp[p][row] = down_e .
 // h_p in f32 (h_p the PH row p). Same launch conditions.
 extern "C" __global__ __launch_bounds__(64 * PH_WAVES) void sepia_ph_down(
     PfProj down, PfProj s_down, int32_t n_routed, int64_t I, int64_t H, const uint8_t *__restrict__ phh,
     const float *__restrict__ phhs, const int32_t *__restrict__ list, const int32_t *__restrict__ units,
     const int32_t *__restrict__ n_units, float *__restrict__ yp) {
-    const PfSlot slot = pf_slot();
+    const PfSlot slot = pf_slot(n_units[0]);
     if (slot.y >= n_units[0]) return;
     extern __shared__ __attribute__((aligned(16))) uint8_t pf_smem[];
-    uint8_t *smem = pf_smem;
     const int32_t *un = units + 3 * slot.y;
     const int32_t e = un[0], nv = un[2];
     const bool routed = e < n_routed;
     const PfProj &D = routed ? down : s_down;
     const int64_t ei = routed ? e : e - n_routed;
     const uint8_t *wd = D.base + ei * D.stride;
-    const int64_t sl = ph_slice(D.type, slot.x);
-    if (sl < 0) return;
-    uint32_t *roff;
+    int64_t *roff;
     int32_t *pair;
     float *srow;
-    pq_unit_rows(list + un[1], nv, false, 1, (I / 256) * PH_REC, phhs, smem, roff, pair, srow);
-    PH_DISPATCH(D.type, false, sl * 128, smem, wd, wd, D.row_bytes, ph_nb(D.type, D.n_blocks), phh,
-                roff, pair, srow, nv, yp, H);
+    ph_unit_rows(list + un[1], nv, false, 1, (I / 128) * PH_REC, phhs, pf_smem, roff, pair, srow);
+    ph_run<false>(D.type, pf_smem, wd, wd, D.row_bytes, ph_nb(D.type, D.n_blocks), phh, roff, pair, srow, nv, slot.x * 256,
+                  H, yp, H);
 }

@@ -167,14 +167,12 @@ static int g_opt_pf_route_m = 1;   /* "pf_route_m": 1 = prefill router logits on
                                     * (sepia_pf_route_m) when x and the router rows are 16-byte aligned
                                     * and hidden is a multiple of 512,
                                     * 0 = sepia_pf_route */
-static int g_opt_pf_h = 1;   /* "pf_h": 1 = a prefill layer whose six projections all have formats of the
-                              * real checkpoint (IQ2_XS, IQ3_XXS, IQ4_XS, Q5_K, Q6_K, Q8_0) runs them on the
-                              * f16 matrix cores (sepia_ph_quant, sepia_ph_gateup, sepia_ph_down); 0 = the
-                              * bf16 kernels */
+static int g_opt_pf_h = 1;   /* "pf_h": 1 = prefill layers with 4-byte-aligned rows that the int8 kernels do
+                              * not take run their projections on the f16 matrix cores (sepia_ph_quant,
+                              * sepia_ph_gateup, sepia_ph_down); 0 = on the bf16 kernels */
 static int g_opt_pf_q = 1;   /* "pf_q": 1 = a prefill layer whose six projections are all Q2_K, Q3_K or Q4_K
                               * runs them on the int8 matrix cores (sepia_pf_quant, sepia_pf_gateup_q,
-                              * sepia_pf_down_q); 0 = the bf16 kernels sepia_pf_gateup / _down, which
-                              * every other layer always takes */
+                              * sepia_pf_down_q); 0 = as any other layer */
 static int g_opt_tile_t = 0; /* sepia_hip_set_option("tile_t", T) forces T steps per workgroup */
 
 /* Geometry for `mats` stacked copies of a [rows, 256 * n_blocks] matrix; 0
@@ -1851,7 +1849,6 @@ int sepia_hip_synth_blocks(int ggml_type, SepiaGpuBuf *buf, size_t off, int64_t 
 
 /* --------------------------------------------------------------- MoE ---- */
 #define RT_THREADS 512   /* threads per router workgroup (RT_NT in kernels/moe.h) */
-#define PH_WAVES 16      /* waves of an f16 projection workgroup (kernels/prefill_h.h) */
 /* Mirrors struct MoeProj in kernels/moe.h field for field. */
 typedef struct {
     const uint8_t *base;
@@ -2081,10 +2078,16 @@ static int pf_type_ok(int t) {
 }
 /* Formats of the int8 prefill projections (kernels/prefill_q.h): Q2_K, Q3_K, Q4_K. */
 static int pf_type_int(int t) { return t == SEPIA_T_Q2_K || t == SEPIA_T_Q3_K || t == 12; }
-/* Formats of the f16 prefill projections (kernels/prefill_h.h): the real
- * checkpoint's IQ2_XS, IQ3_XXS, IQ4_XS, Q5_K, Q6_K and Q8_0. */
+/* Formats of the real checkpoint: IQ2_XS, IQ3_XXS, IQ4_XS, Q5_K, Q6_K and
+ * Q8_0. The f16 prefill projections (kernels/prefill_h.h) take these and
+ * pf_type_ok's. */
 static int pf_type_h(int t) { return t == 17 || t == 18 || t == 23 || t == 13 || t == 14 || t == 8; }
-#define PH_REC 1056   /* bytes of a 256-column PH record (kernels/prefill_h.h) */
+/* As in kernels/prefill_h.h: pairs per unit, bytes of a 128-column record,
+ * threads and LDS of a projection workgroup. */
+#define PH_UM 64
+#define PH_REC 576
+#define PH_THREADS 512
+#define PH_LDS_BYTES 163840
 
 int sepia_gpu_moe_prefill(const SepiaMoeLayerDesc *L, int64_t n_tokens, SepiaGpuBuf *x, SepiaGpuBuf *y,
                           SepiaGpuBuf *route_out) {
@@ -2119,9 +2122,9 @@ int sepia_gpu_moe_prefill(const SepiaMoeLayerDesc *L, int64_t n_tokens, SepiaGpu
     int q_aligned = 1;
     for (int i = 0; i < (ns > 0 ? 6 : 3); i++)
         if (((uintptr_t)ps[i]->base | ps[i]->stride | ps[i]->row_bytes) & 3) q_aligned = 0;
-    /* f16 path: every projection in the real checkpoint's formats, 4-byte
-     * aligned rows (activations as PH rows: kernels/prefill_h.h, 1056 bytes
-     * per 256 columns); Q8_0 has no other prefill kernels */
+    /* every projection in the real checkpoint's formats, 4-byte aligned rows:
+     * the f16 path (activations as PH rows: kernels/prefill_h.h); Q8_0 has no
+     * other prefill kernels, and only such layers may hold it */
     const int use_h_all = g_opt_pf_h && q_aligned && pf_type_h(g.type) && pf_type_h(d.type) &&
                           (ns == 0 || (pf_type_h(sg.type) && pf_type_h(sd.type)));
     for (int i = 0; i < (ns > 0 ? 6 : 3); i++)
@@ -2142,12 +2145,6 @@ int sepia_gpu_moe_prefill(const SepiaMoeLayerDesc *L, int64_t n_tokens, SepiaGpu
         return 0;
     const size_t route_bytes = (size_t)T * (size_t)(tk + n_sel) * 4;
     if (route_out && !chk(route_out, 0, route_bytes, op, "route_out")) return 0;
-    /* units of <= 32 pairs: routed pairs split over at most n_routed experts,
-     * each shared expert takes every token */
-    const int64_t umax = (T * tk + 31) / 32 + nr + (int64_t)ns * ((T + 31) / 32) + 1;
-    /* grid rows of the f16 unit kernels: a multiple of 8, so they deal the
-     * units to the 8 XCDs in turn (kernels/prefill.h pf_slot) */
-    const int64_t ugrid = (umax + 7) & ~(int64_t)7;
     const int64_t P = T * n_sel;
     if (H % 256 || I % 256) {
         LOG("%s: hidden and inter must be multiples of 256", op);
@@ -2159,13 +2156,27 @@ int sepia_gpu_moe_prefill(const SepiaMoeLayerDesc *L, int64_t n_tokens, SepiaGpu
      * columns) */
     const int use_q = g_opt_pf_q && q_aligned && pf_type_int(g.type) && pf_type_int(d.type) &&
                       (ns == 0 || (pf_type_int(sg.type) && pf_type_int(sd.type)));
-    const int use_h = !use_q && use_h_all;
-    const int64_t ldqx = H / 256 * (use_h ? PH_REC : 832), ldqh = I / 256 * (use_h ? PH_REC : 832);
+    /* f16 path: layers of the real checkpoint's formats, and mixes of those
+     * with the int8 ones (moe_prefill of a Q4_K / Q6_K layer at hidden 4096,
+     * 300 tokens: 1.82 ms on the bf16 kernels, 0.59 ms here), rows 4-byte
+     * aligned; the bf16 kernels take what is left, layers with rows at
+     * 2-byte offsets */
+    const int use_h = !use_q && g_opt_pf_h && q_aligned;
     const int use_qh = use_q || use_h;
-    /* the pipelines address activation rows with 32-bit byte offsets */
-    if (ugrid > 65535 || (H + 255) / 256 > MAX_GRID || (uint64_t)T * H * 2 >= (1ull << 32) ||
+    const int64_t ldqx = use_h ? H / 128 * PH_REC : H / 256 * 832, ldqh = use_h ? I / 128 * PH_REC : I / 256 * 832;
+    /* units of <= um pairs: routed pairs split over at most n_routed experts,
+     * each shared expert takes every token */
+    const int64_t um = use_h ? PH_UM : 32;
+    const int64_t umax = (T * tk + um - 1) / um + nr + (int64_t)ns * ((T + um - 1) / um) + 1;
+    /* grid rows of the f16 unit kernels: a multiple of 8, so they deal the
+     * units to the 8 XCDs in turn (kernels/prefill.h pf_slot) */
+    const int64_t ugrid = (umax + 7) & ~(int64_t)7;
+    /* the int8 and bf16 pipelines address activation rows with 32-bit byte
+     * offsets; all paths keep one bound on the batch */
+    const int64_t u32 = (T * tk + 31) / 32 + nr + (int64_t)ns * ((T + 31) / 32) + 1, rec = use_h ? 1056 : 832;
+    if (((u32 + 7) & ~(int64_t)7) > 65535 || (H + 255) / 256 > MAX_GRID || (uint64_t)T * H * 2 >= (1ull << 32) ||
         (uint64_t)P * I * 2 >= (1ull << 32) || (T * H + 255) / 256 > MAX_GRID || P > MAX_GRID ||
-        (use_qh && ((uint64_t)T * ldqx >= (1ull << 32) || (uint64_t)P * ldqh >= (1ull << 32)))) {
+        (use_qh && ((uint64_t)T * (H / 256 * rec) >= (1ull << 32) || (uint64_t)P * (I / 256 * rec) >= (1ull << 32)))) {
         LOG("%s: batch too large", op);
         return 0;
     }
@@ -2185,10 +2196,12 @@ int sepia_gpu_moe_prefill(const SepiaMoeLayerDesc *L, int64_t n_tokens, SepiaGpu
     PF_REGION(o_hl, use_qh ? 0 : P * I * 2);
     PF_REGION(o_pqx, use_qh ? T * ldqx : 0);
     PF_REGION(o_pqxs, use_qh ? T * 4 : 0);
-    PF_REGION(o_hf, use_qh ? P * I * 4 : 0);
     PF_REGION(o_pqh, use_qh ? P * ldqh : 0);
     PF_REGION(o_pqhs, use_qh ? P * 4 : 0);
-    PF_REGION(o_yp, P * H * 4);
+    /* the down launch's partial rows take the place of h in f32, which is
+     * quantized by then */
+    PF_REGION(o_yp, use_qh && I > H ? P * I * 4 : P * H * 4);
+    const size_t o_hf = o_yp;
 #undef PF_REGION
     uint8_t *s = (uint8_t *)scratch(o, op);
     if (!s) return 0;
@@ -2212,32 +2225,34 @@ int sepia_gpu_moe_prefill(const SepiaMoeLayerDesc *L, int64_t n_tokens, SepiaGpu
         return 0;
     void *a_sel[] = { &logits, &rb, &nr32, &ns32, &tk32, &rs, &gsc, &sel_idx, &sel_w };
     if (!launch(K_PF_SELECT, (unsigned)T, 64, a_sel, op)) return 0;
-    void *a_grp[] = { &sel_idx, &tt, &nr32, &ns32, &tk32, &list, &units, &n_units };
+    int32_t um32 = (int32_t)um;
+    void *a_grp[] = { &sel_idx, &tt, &nr32, &ns32, &tk32, &um32, &list, &units, &n_units };
     if (!launch(K_PF_GROUP, 1, 1024, a_grp, op)) return 0;
     if (use_qh) {
         /* int8 (PQ rows) or f16 (PH rows): quantize x, gate/up to f32 h,
-         * quantize h, down to the per-pair partial rows. The f16 gate/up
-         * runs over 64-row slices of I, its down over 128-row slices of H
-         * (a 256-row format takes two slices, in the first half of the
-         * workgroups). */
+         * quantize h, down to the per-pair partial rows. Gate/up runs over
+         * 128-row slices of I, down over 256-row slices of H. */
         void *pqx = s + o_pqx, *pqxs = s + o_pqxs, *hf = s + o_hf, *pqh = s + o_pqh, *pqhs = s + o_pqhs;
         int64_t ldq_x = ldqx, ldq_h = ldqh;
         const int kq = use_q ? K_PF_QUANT : K_PH_QUANT;
-        const unsigned th_p = use_q ? 512 : 64 * PH_WAVES;   /* threads of a projection workgroup */
-        const unsigned gy = (unsigned)(use_q ? umax : ugrid);   /* its units */
         void *a_qx[] = { &x->dev, &hid, &hid, &pqx, &ldq_x, &pqxs };
         if (!launch(kq, (unsigned)T, 256, a_qx, op)) return 0;
-        void *a_gq[] = { (void *)&g, (void *)&u, (void *)&sg, (void *)&su, &nr32, &nsel32, &inter, &hid,
-                         &pqx, &pqxs, &list, &units, &n_units, &hf };
-        if (!launch2(use_q ? K_PF_GATEUP_Q : K_PH_GATEUP, (unsigned)(use_q ? I / 128 : I / 64), gy, th_p,
-                     PF_LDS_BYTES, a_gq, op))
-            return 0;
         void *a_qh[] = { &hf, &inter, &inter, &pqh, &ldq_h, &pqhs };
-        if (!launch(kq, (unsigned)P, 256, a_qh, op)) return 0;
-        void *a_dq[] = { (void *)&d, (void *)&sd, &nr32, &inter, &hid, &pqh, &pqhs, &list, &units, &n_units, &yp };
-        if (!launch2(use_q ? K_PF_DOWN_Q : K_PH_DOWN, (unsigned)(use_q ? H / 256 : H / 128), gy, th_p,
-                     PF_LDS_BYTES, a_dq, op))
-            return 0;
+        if (use_q) {
+            void *a_gq[] = { (void *)&g, (void *)&u, (void *)&sg, (void *)&su, &nr32, &nsel32, &inter, &hid,
+                             &pqx, &pqxs, &list, &units, &n_units, &hf };
+            if (!launch2(K_PF_GATEUP_Q, (unsigned)(I / 128), (unsigned)umax, 512, PF_LDS_BYTES, a_gq, op)) return 0;
+            if (!launch(kq, (unsigned)P, 256, a_qh, op)) return 0;
+            void *a_dq[] = { (void *)&d, (void *)&sd, &nr32, &inter, &hid, &pqh, &pqhs, &list, &units, &n_units, &yp };
+            if (!launch2(K_PF_DOWN_Q, (unsigned)(H / 256), (unsigned)umax, 512, PF_LDS_BYTES, a_dq, op)) return 0;
+        } else {
+            void *a_gu[] = { (void *)&g, (void *)&u, (void *)&sg, (void *)&su, &nr32, &nsel32, &inter, &hid,
+                             &pqx, &pqxs, &list, &units, &n_units, &hf };
+            if (!launch2(K_PH_GATEUP, (unsigned)(I / 128), (unsigned)ugrid, PH_THREADS, PH_LDS_BYTES, a_gu, op)) return 0;
+            if (!launch(kq, (unsigned)P, 256, a_qh, op)) return 0;
+            void *a_dn[] = { (void *)&d, (void *)&sd, &nr32, &inter, &hid, &pqh, &pqhs, &list, &units, &n_units, &yp };
+            if (!launch2(K_PH_DOWN, (unsigned)(H / 256), (unsigned)ugrid, PH_THREADS, PH_LDS_BYTES, a_dn, op)) return 0;
+        }
     } else {
         int64_t nseg = T * H / 16;
         void *a_sp[] = { &x->dev, &nseg, &xh, &xl };
