@@ -7,8 +7,8 @@
 //   y[t] = sum_{k < topk} w[t][k] down_e(silu(gate_e x_t) * up_e x_t)
 //        + sum_s w[t][topk + s] down_s(silu(gate_s x_t) * up_s x_t).
 // Launches:
-//   sepia_pf_route(_m) logits[T][n_routed + n_shared] = x . Rw^T (f32 tiles,
-//                     or the f32 matrix cores)
+//   sepia_pf_route    logits[T][n_routed + n_shared] = x . Rw^T (f32 tiles; on
+//                     the f32 matrix cores: sepia_pf_route_m, _m2)
 //   sepia_pf_select   one wave per token: idx[T][topk], w[T][topk + n_shared]
 //   sepia_pf_group    one workgroup: the (token, slot) pairs p = t * n_sel + k
 //                     sorted by expert (shared expert s is expert
@@ -52,8 +52,8 @@ typedef float pf_f32x4 __attribute__((ext_vector_type(4)));
 // in the real formats: 3.79 -> 3.02 ms when it came in). A few units would
 // leave some XCDs one more each than others (51 units of 24 slices on 32 CUs
 // an XCD: 6 rounds where 5 do; 9 tokens: gate/up 352 -> 328 us), and their
-// rows are few:
-// they keep the launch order, as the int8 kernels do, which measured no better with the dealing (1.90 -> 1.93 ms).
+// rows are few: they keep the launch order, as the int8 kernels do, which
+// measured no better with the dealing (1.90 -> 1.93 ms).
 #define PF_DEAL_UNITS 128
 struct PfSlot {
     int32_t x, y;
@@ -102,73 +102,103 @@ extern "C" __global__ __launch_bounds__(256) void sepia_pf_route(const float *__
         }
 }
 
-// The same logits on the f32 matrix cores: one workgroup of four waves per
-// 16-token x 16-row tile (grid: T / 16 x n_tot / 16), wave w taking the
-// columns [w H / 4, (w + 1) H / 4) in steps of 16 (so 544 tiles of C5 keep
-// every SIMD busy, with a quarter of the dependent MFMA chain each). Lane l
-// loads columns 4 (l >> 4) .. + 3 of the step for token / row l & 15 as one
-// float4; MFMA i of the step takes component i, so the four MFMAs cover the
-// step's 16 columns once each. The four quarter sums are added in LDS in
-// wave order (f32 products, f32 sums; only the summation order differs
-// from sepia_pf_route). Needs x, rw and ld 16-byte aligned and H a multiple
-// of 512 (the host checks).
-typedef float pf_f32x4v __attribute__((ext_vector_type(4)));
-extern "C" __global__ __launch_bounds__(256) void sepia_pf_route_m(const float *__restrict__ x, int64_t T,
-                                                                   const float *__restrict__ rw, int64_t ld,
-                                                                   int64_t n_tot, int64_t H, float *__restrict__ logits) {
-    __shared__ pf_f32x4 part[3][64];
+// The same logits on the f32 matrix cores: a workgroup of W waves per tile of
+// 16 MT tokens x 16 NT rows, 16 W columns (a chunk) per barrier. The chunk's
+// rows go from memory through registers (four chunks ahead) into one of two
+// LDS buffers, as whole 16-byte pieces along the rows; wave w then reads its
+// 16 columns of them as MFMA fragments, lane l columns 4 (l >> 4) .. + 3 of
+// token / row l & 15: MFMA i takes component i, so four MFMAs cover the wave's
+// columns once each. The W partial sums are added in LDS in wave order (f32
+// products, f32 sums; only the summation order differs from sepia_pf_route).
+// Rows are 4 W + 2 pieces apart in LDS, which spreads a fragment read over the
+// banks. Needs x, rw and ld 16-byte aligned and H a multiple of 16 W (the host
+// checks).
+// What bounds it: up to one tile a CU the chain of a tile's chunks, then the
+// rate of the loads. Fragments read straight from memory touch 16 rows an
+// instruction and kept each CU at about 20 bytes a clock (258 rows of 6144:
+// 9 tokens 23 us with four waves, 19 with 16; 512 tokens 61; 1999 tokens 199;
+// through LDS 15, 36 and 132). 2 x 2 tiles halve the loads and win where they
+// still fill the chip (1999 tokens 106; 512 tokens 45, 2 x 1 tiles 40). Error
+// of the sums against 64 bits: 5.0e-7 with eight waves, 6.9e-7 with four.
+template <int MT, int NT, int W>
+__device__ __forceinline__ void pf_route_tiles(const float *__restrict__ x, int64_t T, const float *__restrict__ rw,
+                                               int64_t ld, int64_t n_tot, int64_t H, float *__restrict__ logits) {
+    constexpr int D = 4, J = MT + NT, R = 16 * J, PR = 4 * W, ST = PR + 2;   // PR: pieces of a row per chunk
+    constexpr int n_stage = 2 * R * ST, n_part = W * MT * NT * 64;
+    __shared__ pf_f32x4 lds[n_stage > n_part ? n_stage : n_part];
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63, r = l & 15, g = l >> 4;
-    const int64_t t0 = (int64_t)blockIdx.x * 16, r0 = (int64_t)blockIdx.y * 16;
-    const int64_t t = t0 + r < T ? t0 + r : T - 1, rr = r0 + r < n_tot ? r0 + r : n_tot - 1;
-    const int64_t c0 = (int64_t)w * (H / 4);
-    const pf_f32x4v *xa = (const pf_f32x4v *)(x + t * H + c0) + g, *wa = (const pf_f32x4v *)(rw + rr * ld + c0) + g;
-    pf_f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    // eight steps in registers while the next eight load (n a multiple of 8)
-    const int64_t n = H / 64;
-    pf_f32x4v a[8], b[8];
+    const int64_t t0 = (int64_t)blockIdx.x * (16 * MT), r0 = (int64_t)blockIdx.y * (16 * NT);
+    const pf_f32x4 *src[J];
+    int dst[J];
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
-        a[u] = xa[4 * u];
-        b[u] = wa[4 * u];
+    for (int j = 0; j < J; j++) {
+        const int p = j * 64 * W + threadIdx.x, row = p / PR, c = p % PR;
+        const int64_t t = t0 + row, rr = r0 + row - 16 * MT;
+        src[j] = (const pf_f32x4 *)(row < 16 * MT ? x + (t < T ? t : T - 1) * H : rw + (rr < n_tot ? rr : n_tot - 1) * ld) + c;
+        dst[j] = row * ST + c;
     }
-    for (int64_t k = 0; k < n; k += 8) {
-        pf_f32x4v a2[8], b2[8];
-        const bool more = k + 8 < n;
-        if (more) {
+    const int nc = (int)(H / (16 * W));
+    pf_f32x4 acc[MT][NT] = {}, pre[D][J];
 #pragma unroll
-            for (int u = 0; u < 8; u++) {
-                a2[u] = xa[4 * (k + 8 + u)];
-                b2[u] = wa[4 * (k + 8 + u)];
-            }
-        }
+    for (int d = 0; d < D; d++)
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
+        for (int j = 0; j < J; j++) pre[d][j] = src[j][PR * (d < nc ? d : nc - 1)];
+    for (int c = 0; c < nc; c += D) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i], b[u][i], acc, 0, 0, 0);
-        }
-        if (more) {
+        for (int d = 0; d < D; d++) {
+            pf_f32x4 *buf = lds + (d & 1) * (R * ST);
+            // chunks past the last are zeros (no branch: the loads stay in flight)
 #pragma unroll
-            for (int u = 0; u < 8; u++) {
-                a[u] = a2[u];
-                b[u] = b2[u];
-            }
+            for (int j = 0; j < J; j++) buf[dst[j]] = c + d < nc ? pre[d][j] : pf_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            const int nx = c + d + D < nc ? c + d + D : nc - 1;
+#pragma unroll
+            for (int j = 0; j < J; j++) pre[d][j] = src[j][PR * nx];
+            // a barrier for LDS alone; the next write to this buffer comes after the next one
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+            pf_f32x4 a[MT], b[NT];
+#pragma unroll
+            for (int m = 0; m < MT; m++) a[m] = buf[(16 * m + r) * ST + 4 * w + g];
+#pragma unroll
+            for (int n = 0; n < NT; n++) b[n] = buf[(16 * (MT + n) + r) * ST + 4 * w + g];
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int m = 0; m < MT; m++)
+#pragma unroll
+                    for (int n = 0; n < NT; n++)
+                        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m][i], b[n][i], acc[m][n], 0, 0, 0);
         }
     }
-    // acc[i]: token t0 + 4 g + i, row r0 + r; quarters 1..3 to LDS, added to quarter 0 in order
-    if (w > 0) part[w - 1][l] = acc;
+    // acc[m][n][i]: token t0 + 16 m + 4 g + i, row r0 + 16 n + r
     __syncthreads();
-    if (w > 0) return;
+    float *part = (float *)lds;
 #pragma unroll
-    for (int q = 0; q < 3; q++) {
-        const pf_f32x4 v = part[q][l];
+    for (int m = 0; m < MT; m++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) acc[i] += v[i];
+        for (int n = 0; n < NT; n++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) part[((w * MT + m) * NT + n) * 256 + 16 * (4 * g + i) + r] = acc[m][n][i];
+    __syncthreads();
+    for (int i = threadIdx.x; i < MT * NT * 256; i += 64 * W) {
+        const int q = i >> 8, e = i & 255;
+        float s = part[i];
+#pragma unroll
+        for (int v = 1; v < W; v++) s += part[v * MT * NT * 256 + i];
+        const int64_t t = t0 + 16 * (q / NT) + (e >> 4), ro = r0 + 16 * (q % NT) + (e & 15);
+        if (t < T && ro < n_tot) logits[t * n_tot + ro] = s;
     }
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int64_t tt = t0 + 4 * g + i, ro = r0 + r;
-        if (tt < T && ro < n_tot) logits[tt * n_tot + ro] = acc[i];
-    }
+}
+extern "C" __global__ __launch_bounds__(512, 2) void sepia_pf_route_m(const float *__restrict__ x, int64_t T,
+                                                                      const float *__restrict__ rw, int64_t ld,
+                                                                      int64_t n_tot, int64_t H, float *__restrict__ logits) {
+    pf_route_tiles<1, 1, 8>(x, T, rw, ld, n_tot, H, logits);
+}
+extern "C" __global__ __launch_bounds__(256, 4) void sepia_pf_route_m2(const float *__restrict__ x, int64_t T,
+                                                                       const float *__restrict__ rw, int64_t ld,
+                                                                       int64_t n_tot, int64_t H, float *__restrict__ logits) {
+    pf_route_tiles<2, 2, 4>(x, T, rw, ld, n_tot, H, logits);
 }
 
 // One wave per token (route.h).
@@ -186,53 +216,93 @@ extern "C" __global__ __launch_bounds__(64) void sepia_pf_select(const float *__
 // ------------------------------------------------------------- grouping --
 // One workgroup. Pairs p = t * n_sel + k: expert idx[t][k] for k < topk,
 // n_routed + (k - topk) after. list[] holds the pairs grouped by expert
-// (ascending expert; within an expert in arrival order, which does not
+// (ascending expert; within a routed expert in arrival order, which does not
 // affect any result), units[u] = {expert, first list position, count <=
 // um}, n_units[0] their number. E = n_routed + n_shared <= 1088.
+// What bounds it is the chain of latencies of a single workgroup: four idx
+// loads in flight per thread, the two running sums over the experts as wave
+// scans (two experts a thread), and the shared experts, whose pairs are
+// known without counting, outside the atomics (256 + 2
+// experts, top-6: 9 tokens 16 -> 4 us, 512 tokens 19 -> 5, 1999 tokens 30 ->
+// 11 against one thread summing over the experts).
 extern "C" __global__ __launch_bounds__(1024) void sepia_pf_group(const int32_t *__restrict__ idx, int64_t T,
                                                                   int32_t n_routed, int32_t n_shared, int32_t topk, int32_t um,
                                                                   int32_t *__restrict__ list,
                                                                   int32_t *__restrict__ units,
                                                                   int32_t *__restrict__ n_units) {
-    __shared__ int32_t cnt[1088], off[1089], fill[1088], uoff[1089];
-    const int E = n_routed + n_shared, n_sel = topk + n_shared;
-    const int64_t P = T * n_sel;
-    for (int e = threadIdx.x; e < E; e += blockDim.x) {
-        cnt[e] = 0;
-        fill[e] = 0;
-    }
+    __shared__ int32_t cnt[1088], off[1088], cur[1088], uoff[1088], wsum[2][16];
+    const int E = n_routed + n_shared, n_sel = topk + n_shared, tid = threadIdx.x;
+    const int32_t Pr = (int32_t)(T * topk);   // routed pairs
+    for (int e = tid; e < E; e += 1024) cnt[e] = e < n_routed ? 0 : (int32_t)T;
     __syncthreads();
-    auto expert_of = [&](int64_t p) {
-        const int64_t t = p / n_sel;
-        const int k = (int)(p - t * n_sel);
-        return k < topk ? idx[t * topk + k] : n_routed + (k - topk);
+    // f(q, expert) over the routed pairs q = t * topk + k
+    auto each_routed = [&](auto f) {
+        for (int32_t q0 = tid; q0 < Pr; q0 += 4096) {
+            int32_t e[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) e[u] = idx[q0 + 1024 * u < Pr ? q0 + 1024 * u : Pr - 1];
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (q0 + 1024 * u < Pr) f(q0 + 1024 * u, e[u]);
+        }
     };
-    for (int64_t p = threadIdx.x; p < P; p += blockDim.x) atomicAdd(&cnt[expert_of(p)], 1);
+    each_routed([&](int32_t, int32_t e) { atomicAdd(&cnt[e], 1); });
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int a = 0, u = 0;
-        for (int e = 0; e < E; e++) {
-            off[e] = a;
-            uoff[e] = u;
-            a += cnt[e];
-            u += (cnt[e] + um - 1) / um;
+    // exclusive sums of the pairs and units over the experts
+    const int e0 = 2 * tid, lane = tid & 63, wave = tid >> 6;
+    const int32_t c0 = e0 < E ? cnt[e0] : 0, c1 = e0 + 1 < E ? cnt[e0 + 1] : 0;
+    const int32_t u0 = (c0 + um - 1) / um, u1 = (c1 + um - 1) / um;
+    int32_t a = c0 + c1, b = u0 + u1;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int32_t pa = __shfl_up(a, d, 64), pb = __shfl_up(b, d, 64);
+        if (lane >= d) {
+            a += pa;
+            b += pb;
         }
-        off[E] = a;
-        uoff[E] = u;
-        n_units[0] = u;
+    }
+    if (lane == 63) {
+        wsum[0][wave] = a;
+        wsum[1][wave] = b;
     }
     __syncthreads();
-    for (int64_t p = threadIdx.x; p < P; p += blockDim.x) {
-        const int e = expert_of(p);
-        list[off[e] + atomicAdd(&fill[e], 1)] = (int32_t)p;
-    }
-    for (int e = threadIdx.x; e < E; e += blockDim.x) {
-        for (int j = 0; j < (cnt[e] + um - 1) / um; j++) {
-            int32_t *un = units + 3 * (uoff[e] + j);
-            un[0] = e;
-            un[1] = off[e] + um * j;
-            un[2] = cnt[e] - um * j < um ? cnt[e] - um * j : um;
+    int32_t before_a = 0, before_b = 0, all_b = 0;
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+        if (v < wave) {
+            before_a += wsum[0][v];
+            before_b += wsum[1][v];
         }
+        all_b += wsum[1][v];
+    }
+    a += before_a - c0 - c1;
+    b += before_b - u0 - u1;
+    if (e0 < E) {
+        off[e0] = cur[e0] = a;
+        uoff[e0] = b;
+    }
+    if (e0 + 1 < E) {
+        off[e0 + 1] = cur[e0 + 1] = a + c0;
+        uoff[e0 + 1] = b + u0;
+    }
+    if (tid == 0) n_units[0] = all_b;
+    __syncthreads();
+    each_routed([&](int32_t q, int32_t e) {
+        const uint32_t t = (uint32_t)q / (uint32_t)topk;
+        list[atomicAdd(&cur[e], 1)] = (int32_t)(t * (uint32_t)n_sel) + q - (int32_t)(t * (uint32_t)topk);
+    });
+    auto unit = [&](int e, int j) {
+        int32_t *un = units + 3 * (uoff[e] + j);
+        un[0] = e;
+        un[1] = off[e] + um * j;
+        un[2] = cnt[e] - um * j < um ? cnt[e] - um * j : um;
+    };
+    for (int e = tid; e < n_routed; e += 1024)
+        for (int j = 0; j < (cnt[e] + um - 1) / um; j++) unit(e, j);
+    for (int s = 0; s < n_shared; s++) {
+        const int e = n_routed + s;
+        for (int32_t t = tid; t < (int32_t)T; t += 1024) list[off[e] + t] = t * n_sel + topk + s;
+        for (int j = tid; j < (cnt[e] + um - 1) / um; j += 1024) unit(e, j);
     }
 }
 

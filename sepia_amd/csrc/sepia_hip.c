@@ -60,7 +60,7 @@ enum {
     /* batched prefill MoE layer (kernels/prefill.h) */
     K_PF_ROUTE = K_MQ_DN + 1, K_PF_SELECT, K_PF_GROUP, K_PF_GATEUP, K_PF_DOWN, K_PF_COMBINE, K_PF_SPLIT,
     /* prefill router logits on the f32 matrix cores (kernels/prefill.h) */
-    K_PF_ROUTE_M,
+    K_PF_ROUTE_M, K_PF_ROUTE_M2,
     /* u32 fill (counter words of caller-provided scratch) */
     K_FILL_U32,
     /* attention (kernels/attn.h): relative-position projection, banded attention and the fold of its splits */
@@ -94,7 +94,7 @@ static const char *const k_names[K_COUNT] = {
     "sepia_mq_mv_q5_k", "sepia_mq_mv_q6_k", "sepia_mq_mv_iq4_xs", "sepia_mq_mv_q8_0",
     "sepia_mq_gateup", "sepia_mq_down",
     "sepia_pf_route", "sepia_pf_select", "sepia_pf_group", "sepia_pf_gateup", "sepia_pf_down", "sepia_pf_combine",
-    "sepia_pf_split", "sepia_pf_route_m", "sepia_fill_u32",
+    "sepia_pf_split", "sepia_pf_route_m", "sepia_pf_route_m2", "sepia_fill_u32",
     "sepia_rel_project_f32", "sepia_attn_bounds", "sepia_attn_wave", "sepia_attn_wave_d",
     "sepia_attn_tile", "sepia_attn_tile_d", "sepia_attn_combine",
     "sepia_pf_quant", "sepia_pf_gateup_q", "sepia_pf_down_q",
@@ -164,9 +164,8 @@ static int g_mq_kind = 0;          /* the launch kind mq_geo is planning: 1 matv
 static int g_opt_mq_x = 0;   /* "mq_x": 0 = planner's choice, 1 = vector from global, 2 = vector by LDS DMA,
                               * 3 = converter waves */
 static int g_opt_pf_route_m = 1;   /* "pf_route_m": 1 = prefill router logits on the f32 matrix cores
-                                    * (sepia_pf_route_m) when x and the router rows are 16-byte aligned
-                                    * and hidden is a multiple of 512,
-                                    * 0 = sepia_pf_route */
+                                    * (sepia_pf_route_m, _m2) when x and the router rows are 16-byte
+                                    * aligned, 0 = sepia_pf_route */
 static int g_opt_pf_h = 1;   /* "pf_h": 1 = prefill layers with 4-byte-aligned rows that the int8 kernels do
                               * not take run their projections on the f16 matrix cores (sepia_ph_quant,
                               * sepia_ph_gateup, sepia_ph_down); 0 = on the bf16 kernels */
@@ -2219,9 +2218,14 @@ int sepia_gpu_moe_prefill(const SepiaMoeLayerDesc *L, int64_t n_tokens, SepiaGpu
     float rs = L->route_scale, gsc = L->global_scale;
     int32_t nr32 = nr, ns32 = ns, tk32 = tk, nsel32 = n_sel;
     void *a_rt[] = { &x->dev, &tt, &rw, &ld, &ntot, &hid, &logits };
-    const int rt_m = g_opt_pf_route_m && ((((uintptr_t)x->dev | (uintptr_t)rw) & 15) == 0) && (ld % 4) == 0 && H % 512 == 0;
-    if (rt_m ? !launch2(K_PF_ROUTE_M, (unsigned)((T + 15) / 16), (unsigned)((n_tot + 15) / 16), 256, 0, a_rt, op)
-             : !launch2(K_PF_ROUTE, (unsigned)((T + 31) / 32), (unsigned)((n_tot + 31) / 32), 256, 0, a_rt, op))
+    /* 16 x 16 tiles up to 4.5 a CU, 32 x 32 tiles beyond (258 rows of 6144:
+     * 512 tokens 36 us against 45, 1024 tokens, 1088 tiles, 61 against 73, 1200
+     * tokens 81 against 74, 1999 tokens 132 against 106) */
+    const int rt_m = g_opt_pf_route_m && ((((uintptr_t)x->dev | (uintptr_t)rw) & 15) == 0);
+    const int64_t t16 = (T + 15) / 16, r16 = (n_tot + 15) / 16, t32 = (T + 31) / 32, r32 = (n_tot + 31) / 32;
+    if (!rt_m                ? !launch2(K_PF_ROUTE, (unsigned)t32, (unsigned)r32, 256, 0, a_rt, op)
+        : t16 * r16 <= 1152 ? !launch2(K_PF_ROUTE_M, (unsigned)t16, (unsigned)r16, 512, 0, a_rt, op)
+                            : !launch2(K_PF_ROUTE_M2, (unsigned)t32, (unsigned)r32, 256, 0, a_rt, op))
         return 0;
     void *a_sel[] = { &logits, &rb, &nr32, &ns32, &tk32, &rs, &gsc, &sel_idx, &sel_w };
     if (!launch(K_PF_SELECT, (unsigned)T, 64, a_sel, op)) return 0;
