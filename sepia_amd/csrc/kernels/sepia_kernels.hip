@@ -164,8 +164,59 @@ __device__ __forceinline__ float block_max_256(float v, float *lds4) {
     return fmaxf(fmaxf(lds4[0], lds4[1]), fmaxf(lds4[2], lds4[3]));
 }
 
-// y[r,i] = w[i] * (x[r,i] * (1 / sqrt(mean(x^2) + eps))): one workgroup per row
+// y[r,i] = w[i] * (x[r,i] * (1 / sqrt(mean(x^2) + eps))), y may be x
 // (reference src/sepia.c:719-729 order: x * inv first, then * w).
+// What bounds it is one row's chain: load, sum, store. Rows of n % 4 == 0
+// floats with w, x and y on 16 bytes (the host checks) load both as float4
+// before the sum and keep them for the store (one row of 6144, then 72 of
+// 128 as q and k norm in an attention block: 29 us for the three launches
+// with 256 threads a row and scalar loads, 12 so):
+//   sepia_rmsnorm_wave  n <= 512: a wave per row, four rows per workgroup,
+//                       no barrier
+//   sepia_rmsnorm_row   longer: a workgroup per row, two float4 a thread up
+//                       to 8192 floats (blockDim: host), the rest in a loop
+//   sepia_rmsnorm_f32   any alignment and n: a workgroup per row
+__device__ __forceinline__ float rms_sq(float4 v, float s) {
+    return __builtin_fmaf(v.w, v.w, __builtin_fmaf(v.z, v.z, __builtin_fmaf(v.y, v.y, __builtin_fmaf(v.x, v.x, s))));
+}
+__device__ __forceinline__ float4 rms_out(float4 w, float4 x, float inv) {
+    return make_float4(w.x * (x.x * inv), w.y * (x.y * inv), w.z * (x.z * inv), w.w * (x.w * inv));
+}
+extern "C" __global__ __launch_bounds__(256) void sepia_rmsnorm_wave(
+    const float *w, const float *x, float *y, int64_t n, float eps, int64_t rows) {
+    const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (r >= rows) return;
+    const int n4 = (int)(n >> 2), l = threadIdx.x & 63, i0 = l < n4 ? l : 0, i1 = l + 64 < n4 ? l + 64 : 0;
+    const float4 *xr = (const float4 *)(x + r * n);
+    float4 *yr = (float4 *)(y + r * n);
+    const float4 x0 = xr[i0], x1 = xr[i1], w0 = ((const float4 *)w)[i0], w1 = ((const float4 *)w)[i1];
+    float s = l < n4 ? rms_sq(x0, 0.0f) : 0.0f;
+    if (l + 64 < n4) s = rms_sq(x1, s);
+    const float inv = 1.0f / sqrtf(wave_sum(s) / (float)n + eps);
+    if (l < n4) yr[l] = rms_out(w0, x0, inv);
+    if (l + 64 < n4) yr[l + 64] = rms_out(w1, x1, inv);
+}
+extern "C" __global__ __launch_bounds__(1024) void sepia_rmsnorm_row(
+    const float *w, const float *x, float *y, int64_t n, float eps) {
+    __shared__ float red[16];
+    const int64_t n4 = n >> 2, nt = blockDim.x, i0 = threadIdx.x, i1 = i0 + nt;
+    const float4 *xr = (const float4 *)(x + (int64_t)blockIdx.x * n), *w4 = (const float4 *)w;
+    float4 *yr = (float4 *)(y + (int64_t)blockIdx.x * n);
+    const float4 x0 = xr[i0 < n4 ? i0 : 0], x1 = xr[i1 < n4 ? i1 : 0];
+    const float4 w0 = w4[i0 < n4 ? i0 : 0], w1 = w4[i1 < n4 ? i1 : 0];
+    float s = i0 < n4 ? rms_sq(x0, 0.0f) : 0.0f;
+    if (i1 < n4) s = rms_sq(x1, s);
+    for (int64_t i = i1 + nt; i < n4; i += nt) s = rms_sq(xr[i], s);
+    s = wave_sum(s);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    s = red[0];
+    for (int v = 1; v < (int)(nt >> 6); v++) s += red[v];
+    const float inv = 1.0f / sqrtf(s / (float)n + eps);
+    if (i0 < n4) yr[i0] = rms_out(w0, x0, inv);
+    if (i1 < n4) yr[i1] = rms_out(w1, x1, inv);
+    for (int64_t i = i1 + nt; i < n4; i += nt) yr[i] = rms_out(w4[i], xr[i], inv);
+}
 extern "C" __global__ __launch_bounds__(256) void sepia_rmsnorm_f32(
     const float *w, const float *x, float *y, int64_t n, float eps) {
     __shared__ float red[4];

@@ -46,7 +46,7 @@ enum {
     K_DQ_IQ2_XXS, K_DQ_IQ2_XS, K_DQ_IQ3_XXS, K_DQ_IQ4_XS, K_DQ_F16,
     K_MV_Q8_0, K_MV_Q2_K, K_MV_Q3_K, K_MV_Q4_K, K_MV_Q5_K, K_MV_Q6_K,
     K_MV_IQ2_XXS, K_MV_IQ2_XS, K_MV_IQ3_XXS, K_MV_IQ4_XS,
-    K_MATVEC_F32, K_SILU_MUL, K_ADD, K_SCALE, K_COPY, K_TOUCH, K_RMSNORM, K_SOFTMAX,
+    K_MATVEC_F32, K_SILU_MUL, K_ADD, K_SCALE, K_COPY, K_TOUCH, K_RMSNORM, K_RMSNORM_WAVE, K_RMSNORM_ROW, K_SOFTMAX,
     K_SCONV, K_SCONV_HIST, K_MOE_ROUTE, K_MOE_GATEUP, K_MOE_DOWN, K_SYNTH_FILL, K_SYNTH_F16,
     K_TILE_Q2_K, K_TILE_Q3_K, K_TILE_Q4_K,
     /* expert-FFN tile kernels: 9 (routed, shared) format pairs over
@@ -84,7 +84,8 @@ static const char *const k_names[K_COUNT] = {
     "sepia_matvec_generic_iq2_xxs", "sepia_matvec_generic_iq2_xs", "sepia_matvec_generic_iq3_xxs",
     "sepia_matvec_generic_iq4_xs",
     "sepia_matvec_f32", "sepia_silu_mul_f32", "sepia_add_f32", "sepia_scale_f32", "sepia_copy_f32",
-    "sepia_touch_f32", "sepia_rmsnorm_f32", "sepia_softmax_f32", "sepia_sconv_f32",
+    "sepia_touch_f32", "sepia_rmsnorm_f32", "sepia_rmsnorm_wave", "sepia_rmsnorm_row", "sepia_softmax_f32",
+    "sepia_sconv_f32",
     "sepia_sconv_hist_roll_f32", "sepia_moe_route", "sepia_moe_gateup_generic", "sepia_moe_down_generic",
     "sepia_synth_fill", "sepia_synth_patch_f16",
     "sepia_mv_q2_k", "sepia_mv_q3_k", "sepia_mv_q4_k",
@@ -1020,8 +1021,13 @@ static int do_rmsnorm(const char *op, SepiaGpuBuf *w, size_t w_off, SepiaGpuBuf 
         return 0;
     if (!need_batch(op) || !prep_in_r(w, w_off, (size_t)n * 4, op) || !prep_in(x, op) || !prep_out(y, op)) return 0;
     const float *wp = (const float *)(w->dev + w_off);
-    void *args[] = { &wp, &x->dev, &y->dev, &n, &eps };
-    return launch(K_RMSNORM, (unsigned)rows, 256, args, op);
+    void *args[] = { &wp, &x->dev, &y->dev, &n, &eps, &rows };
+    if ((((uintptr_t)wp | (uintptr_t)x->dev | (uintptr_t)y->dev) & 15) || n % 4)
+        return launch(K_RMSNORM, (unsigned)rows, 256, args, op);
+    if (n <= 512) return launch(K_RMSNORM_WAVE, (unsigned)((rows + 3) / 4), 256, args, op);
+    /* two float4 a thread, so the row stays in registers up to 8192 floats */
+    const int64_t waves = (n / 4 + 127) / 128;
+    return launch(K_RMSNORM_ROW, (unsigned)rows, waves < 16 ? (unsigned)waves * 64 : 1024, args, op);
 }
 
 int sepia_gpu_rmsnorm(SepiaGpuBuf *w, SepiaGpuBuf *x, SepiaGpuBuf *y, int64_t rows, int64_t n, float eps) {
