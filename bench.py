@@ -240,7 +240,7 @@ MEASURED_TRAFFIC_C2 = {"sepia_mq_gateup": 13001871, "sepia_mq_down": 8582520}
 MEASURED_TRAFFIC_C3 = {"sepia_moe_route": 6612357, "sepia_mq_gateup": 122283851, "sepia_mq_down": 72124327}
 MEASURED_TRAFFIC_REAL = {"sepia_moe_route": 6612386, "sepia_mq_gateup": 118571552, "sepia_mq_down": 76561443}
 MEASURED_TRAFFIC_C5 = {"sepia_pf_gateup_q": 2999146132, "sepia_pf_down_q": 1900014470}
-MEASURED_TRAFFIC_C5_REAL = {"sepia_ph_gateup": 3364945920, "sepia_ph_down": 2298700800}   # moe_prefill_c5_real_counters.md
+MEASURED_TRAFFIC_C5_REAL = {"sepia_ph_gateup": 2848514048, "sepia_ph_down": 2133344256}   # moe_prefill_c5_real_counters.md
 
 
 def cpu_sample(fn, min_seconds, max_calls):
