@@ -82,7 +82,8 @@ int sepia_hip_moe_decode_noalloc(const SepiaMoeLayerDesc *layer, SepiaGpuBuf *x,
  * (without Q8_0) on the f16 ones (weights as exact f16 integer codes,
  * activations as f16 hi + lo planes), all with f32 accumulation. Rows 4-byte
  * aligned; layers with rows at 2-byte offsets (without Q8_0) run on the bf16
- * ones (weights and activations as bf16 hi + lo pairs). x, y: f32
+ * ones (weights and activations as bf16 hi + lo pairs), and so do layers of
+ * both kinds whose f16 scratch a capture does not hold. x, y: f32
  * [n_tokens][hidden] at offset 0.
  * route_out (optional): int32 idx[n_tokens][topk] followed by f32
  * w[n_tokens][topk + n_shared]. */

@@ -2094,6 +2094,51 @@ static int pf_type_h(int t) { return t == 17 || t == 18 || t == 23 || t == 13 ||
 #define PH_THREADS 512
 #define PH_LDS_BYTES 163840
 
+/* Units of <= um pairs at most: routed pairs split over at most n_routed
+ * experts, each shared expert takes every token. */
+static int64_t pf_units(int64_t T, int64_t tk, int64_t nr, int64_t ns, int64_t um) {
+    return (T * tk + um - 1) / um + nr + ns * ((T + um - 1) / um) + 1;
+}
+/* rows records of n columns, rec bytes per 256, pass 32-bit byte offsets */
+static int pf_rows_large(int64_t rows, int64_t n, int64_t rec) {
+    return (uint64_t)rows * (uint64_t)(n / 256 * rec) >= (1ull << 32);
+}
+/* the f16 path's bound: of two planes and eight f32 sums (its kernels use
+ * 64-bit offsets, so its larger records may pass it) */
+#define PF_HREC 1056
+
+/* Regions of a call's scratch; rec: bytes of a 256-column record of the int8
+ * or f16 path, 0 for the bf16 path. */
+typedef struct {
+    size_t logits, idx, w, list, units, nu, xh, xl, hh, hl, pqx, pqxs, pqh, pqhs, yp, bytes;
+} PfScratch;
+static PfScratch pf_scratch(int64_t T, int64_t H, int64_t I, int64_t n_tot, int64_t tk, int64_t n_sel, int64_t umax,
+                            int64_t rec) {
+    const int64_t P = T * n_sel;
+    PfScratch o;
+    memset(&o, 0, sizeof o);
+#define PF_REGION(name, n) o.name = o.bytes, o.bytes += ((size_t)(n) + 255) & ~(size_t)255
+    PF_REGION(logits, T * n_tot * 4);
+    PF_REGION(idx, T * tk * 4);
+    PF_REGION(w, P * 4);
+    PF_REGION(list, P * 4);
+    PF_REGION(units, umax * 12);
+    PF_REGION(nu, 4);   /* n_units */
+    PF_REGION(xh, rec ? 0 : T * H * 2);
+    PF_REGION(xl, rec ? 0 : T * H * 2);
+    PF_REGION(hh, rec ? 0 : P * I * 2);
+    PF_REGION(hl, rec ? 0 : P * I * 2);
+    PF_REGION(pqx, T * (H / 256 * rec));
+    PF_REGION(pqxs, rec ? T * 4 : 0);
+    PF_REGION(pqh, P * (I / 256 * rec));
+    PF_REGION(pqhs, rec ? P * 4 : 0);
+    /* the down launch's partial rows take the place of h in f32, which is
+     * quantized by then */
+    PF_REGION(yp, rec && I > H ? P * I * 4 : P * H * 4);
+#undef PF_REGION
+    return o;
+}
+
 int sepia_gpu_moe_prefill(const SepiaMoeLayerDesc *L, int64_t n_tokens, SepiaGpuBuf *x, SepiaGpuBuf *y,
                           SepiaGpuBuf *route_out) {
     const char *op = "moe_prefill";
@@ -2164,56 +2209,40 @@ int sepia_gpu_moe_prefill(const SepiaMoeLayerDesc *L, int64_t n_tokens, SepiaGpu
     /* f16 path: layers of the real checkpoint's formats, and mixes of those
      * with the int8 ones (moe_prefill of a Q4_K / Q6_K layer at hidden 4096,
      * 300 tokens: 1.82 ms on the bf16 kernels, 0.59 ms here), rows 4-byte
-     * aligned; the bf16 kernels take what is left, layers with rows at
-     * 2-byte offsets */
-    const int use_h = !use_q && g_opt_pf_h && q_aligned;
+     * aligned; the bf16 kernels take what is left: layers with rows at 2-byte
+     * offsets, and mixes whose activation records pass the bound below, with
+     * a matrix that the f16 kernels' 32-bit row offsets do not span, or whose
+     * scratch (more than the bf16 path's) a capture does not hold */
+    int use_h = !use_q && g_opt_pf_h && q_aligned, span = 1;
+    for (int i = 0; i < (ns > 0 ? 6 : 3); i++)
+        if ((uint64_t)(i % 3 == 2 ? H : I) * ps[i]->row_bytes >= (1ull << 32)) span = 0;
+    if (use_h && !use_h_all &&
+        (!span || pf_rows_large(T, H, PF_HREC) || pf_rows_large(P, I, PF_HREC) ||
+         pf_scratch(T, H, I, n_tot, tk, n_sel, pf_units(T, tk, nr, ns, PH_UM), PH_REC * 2).bytes > scratch_limit()))
+        use_h = 0;
     const int use_qh = use_q || use_h;
-    const int64_t ldqx = use_h ? H / 128 * PH_REC : H / 256 * 832, ldqh = use_h ? I / 128 * PH_REC : I / 256 * 832;
-    /* units of <= um pairs: routed pairs split over at most n_routed experts,
-     * each shared expert takes every token */
-    const int64_t um = use_h ? PH_UM : 32;
-    const int64_t umax = (T * tk + um - 1) / um + nr + (int64_t)ns * ((T + um - 1) / um) + 1;
+    const int64_t rec = use_h ? PH_REC * 2 : 832, ldqx = H / 256 * rec, ldqh = I / 256 * rec;
+    const int64_t um = use_h ? PH_UM : 32, umax = pf_units(T, tk, nr, ns, um);
     /* grid rows of the f16 unit kernels: a multiple of 8, so they deal the
      * units to the 8 XCDs in turn (kernels/prefill.h pf_slot) */
     const int64_t ugrid = (umax + 7) & ~(int64_t)7;
     /* the int8 and bf16 pipelines address activation rows with 32-bit byte
      * offsets; all paths keep one bound on the batch */
-    const int64_t u32 = (T * tk + 31) / 32 + nr + (int64_t)ns * ((T + 31) / 32) + 1, rec = use_h ? 1056 : 832;
-    if (((u32 + 7) & ~(int64_t)7) > 65535 || (H + 255) / 256 > MAX_GRID || (uint64_t)T * H * 2 >= (1ull << 32) ||
-        (uint64_t)P * I * 2 >= (1ull << 32) || (T * H + 255) / 256 > MAX_GRID || P > MAX_GRID ||
-        (use_qh && ((uint64_t)T * (H / 256 * rec) >= (1ull << 32) || (uint64_t)P * (I / 256 * rec) >= (1ull << 32)))) {
+    if (((pf_units(T, tk, nr, ns, 32) + 7) & ~(int64_t)7) > 65535 || (H + 255) / 256 > MAX_GRID ||
+        (uint64_t)T * H * 2 >= (1ull << 32) || (uint64_t)P * I * 2 >= (1ull << 32) || (T * H + 255) / 256 > MAX_GRID || P > MAX_GRID ||
+        (use_qh && (pf_rows_large(T, H, use_h ? PF_HREC : 832) || pf_rows_large(P, I, use_h ? PF_HREC : 832)))) {
         LOG("%s: batch too large", op);
         return 0;
     }
     if (!need_batch(op)) return 0;
 
-    size_t o = 0;
-#define PF_REGION(name, bytes) const size_t name = o; o += ((size_t)(bytes) + 255) & ~(size_t)255
-    PF_REGION(o_logits, T * n_tot * 4);
-    PF_REGION(o_idx, T * tk * 4);
-    PF_REGION(o_w, P * 4);
-    PF_REGION(o_list, P * 4);
-    PF_REGION(o_units, umax * 12);
-    PF_REGION(o_nu, 4);   /* n_units */
-    PF_REGION(o_xh, use_qh ? 0 : T * H * 2);
-    PF_REGION(o_xl, use_qh ? 0 : T * H * 2);
-    PF_REGION(o_hh, use_qh ? 0 : P * I * 2);
-    PF_REGION(o_hl, use_qh ? 0 : P * I * 2);
-    PF_REGION(o_pqx, use_qh ? T * ldqx : 0);
-    PF_REGION(o_pqxs, use_qh ? T * 4 : 0);
-    PF_REGION(o_pqh, use_qh ? P * ldqh : 0);
-    PF_REGION(o_pqhs, use_qh ? P * 4 : 0);
-    /* the down launch's partial rows take the place of h in f32, which is
-     * quantized by then */
-    PF_REGION(o_yp, use_qh && I > H ? P * I * 4 : P * H * 4);
-    const size_t o_hf = o_yp;
-#undef PF_REGION
-    uint8_t *s = (uint8_t *)scratch(o, op);
+    const PfScratch o = pf_scratch(T, H, I, n_tot, tk, n_sel, umax, use_qh ? rec : 0);
+    uint8_t *s = (uint8_t *)scratch(o.bytes, op);
     if (!s) return 0;
-    float *logits = (float *)(s + o_logits), *sel_w = (float *)(s + o_w), *yp = (float *)(s + o_yp);
-    void *xh = s + o_xh, *xl = s + o_xl, *hh = s + o_hh, *hl = s + o_hl;
-    int32_t *sel_idx = (int32_t *)(s + o_idx), *list = (int32_t *)(s + o_list), *units = (int32_t *)(s + o_units),
-            *n_units = (int32_t *)(s + o_nu);
+    float *logits = (float *)(s + o.logits), *sel_w = (float *)(s + o.w), *yp = (float *)(s + o.yp);
+    void *xh = s + o.xh, *xl = s + o.xl, *hh = s + o.hh, *hl = s + o.hl;
+    int32_t *sel_idx = (int32_t *)(s + o.idx), *list = (int32_t *)(s + o.list), *units = (int32_t *)(s + o.units),
+            *n_units = (int32_t *)(s + o.nu);
 
     if (!prep_layer(L, &g, &u, &d, &sg, &su, &sd, x, (size_t)T * H * 4, op)) return 0;
     if (!prep_out(y, op) || (route_out && !prep_out(route_out, op))) return 0;
@@ -2242,7 +2271,7 @@ int sepia_gpu_moe_prefill(const SepiaMoeLayerDesc *L, int64_t n_tokens, SepiaGpu
         /* int8 (PQ rows) or f16 (PH rows): quantize x, gate/up to f32 h,
          * quantize h, down to the per-pair partial rows. Gate/up runs over
          * 128-row slices of I, down over 256-row slices of H. */
-        void *pqx = s + o_pqx, *pqxs = s + o_pqxs, *hf = s + o_hf, *pqh = s + o_pqh, *pqhs = s + o_pqhs;
+        void *pqx = s + o.pqx, *pqxs = s + o.pqxs, *hf = s + o.yp, *pqh = s + o.pqh, *pqhs = s + o.pqhs;
         int64_t ldq_x = ldqx, ldq_h = ldqh;
         const int kq = use_q ? K_PF_QUANT : K_PH_QUANT;
         void *a_qx[] = { &x->dev, &hid, &hid, &pqx, &ldq_x, &pqxs };
