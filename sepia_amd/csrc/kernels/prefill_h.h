@@ -132,11 +132,14 @@ extern "C" __global__ __launch_bounds__(256) void sepia_ph_quant(const float *__
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
     m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    // s = 2^e > m (exact scaling): e = the exponent of m's leading bit + 1
+    // s = 2^e > m (exact scaling): e = the exponent of m's leading bit + 1,
+    // held to where s and 1 / s are both normal floats. 2^127 <= m: |v'| < 2,
+    // still exact in f16 hi + lo. m < 2^-126: every v is a multiple of 2^-149,
+    // every v' one of 2^-23, exact too.
     const bool fin = m <= 3.0e38f;
     int e = 0;
     if (fin && m > 0.0f) (void)frexpf(m, &e);
-    e = e < 127 ? e : 127;   // 2^127 <= m < 2^128: |v'| < 2, still exact in f16 hi + lo
+    e = e < -126 ? -126 : e < 127 ? e : 127;
     const float s = !fin ? INFINITY : ldexpf(1.0f, e), inv = fin ? ldexpf(1.0f, -e) : 0.0f;
     if (threadIdx.x == 0) scale[r] = s;
     uint8_t *out = rec + r * ldr;
