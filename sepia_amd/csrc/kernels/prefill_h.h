@@ -122,11 +122,13 @@ extern "C" __global__ __launch_bounds__(256) void sepia_ph_quant(const float *__
     __shared__ float red[4];
     const int64_t r = blockIdx.x;
     const float *row = src + r * ld;
+    // (each times zero: 0, or NaN for a NaN or an infinity; a plain sum of
+    // large finite values could overflow into one)
     float m = 0.0f;
     for (int64_t c = 4 * (int64_t)threadIdx.x; c < K; c += 1024) {
         const float4 v = *(const float4 *)(row + c);
         m = mq_nonfinite_max(fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)))),
-                             (v.x + v.y) + (v.z + v.w));
+                             (v.x * 0.0f + v.y * 0.0f) + (v.z * 0.0f + v.w * 0.0f));
     }
     m = pq_wave_max(m);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
@@ -136,7 +138,7 @@ extern "C" __global__ __launch_bounds__(256) void sepia_ph_quant(const float *__
     // held to where s and 1 / s are both normal floats. 2^127 <= m: |v'| < 2,
     // still exact in f16 hi + lo. m < 2^-126: every v is a multiple of 2^-149,
     // every v' one of 2^-23, exact too.
-    const bool fin = m <= 3.0e38f;
+    const bool fin = m < INFINITY;
     int e = 0;
     if (fin && m > 0.0f) (void)frexpf(m, &e);
     e = e < -126 ? -126 : e < 127 ? e : 127;

@@ -1,10 +1,11 @@
 """The f16 prefill path's row scales: rows whose largest magnitude is a
-denormal. One routed and one shared expert, so that h of either follows from
-two of the oracle's matvecs; each token against the oracle's layer."""
+denormal or close to the largest float. One routed and one shared expert, so
+that h of either follows from two of the oracle's matvecs; each token against
+the oracle's layer."""
 import numpy as np
 import pytest
 
-from sepia_amd import hip
+from sepia_amd import hip, synth
 from test_gpu_parity import Launches, check_route, make_layer, run_prefill
 
 pytestmark = pytest.mark.gpu
@@ -25,6 +26,15 @@ def layer(dev, rng, types):
     spec["router_w"][:] = 0.0   # both experts weigh the same, whatever x
     dev.upload(bufs["rw"], spec["router_w"])
     return desc, spec, bufs
+
+
+def rescale(dev, spec, bufs, name, t, factor):
+    """The f16 scales of a projection's blocks times a factor."""
+    blocks = spec[name][0].reshape(-1, synth.GEOM[t][1])
+    for off in synth.F16_FIELDS[t]:
+        f = blocks[:, off:off + 2].copy().view(np.float16) * np.float16(factor)
+        blocks[:, off:off + 2] = f.view(np.uint8).reshape(-1, 2)
+    dev.upload(bufs[name], spec[name][0])
 
 
 def gate_up(orc, spec, x):
@@ -66,5 +76,32 @@ def test_tiny_rows(dev, orc, types):
         slack = 2.0 ** -149 * (2 * float(np.dot(w[t], sums)) + 2 * float(w[t].sum()) + 4)
         err = np.abs(y[t].astype(np.float64) - y_ref).max()
         assert err <= 2e-5 * np.abs(y_ref).max() + slack, (t, err)
+    for b in bufs.values():
+        dev.free(b)
+
+
+@pytest.mark.parametrize("types", TYPES, ids=str)
+def test_huge_rows(dev, orc, types):
+    """x scaled so that h's largest magnitude comes close to the largest float, and down weights small enough for a
+    finite y."""
+    rng = np.random.default_rng(sum(types) + 1)
+    desc, spec, bufs = layer(dev, rng, types)
+    rescale(dev, spec, bufs, "down", types[1], 2.0 ** -8)
+    rescale(dev, spec, bufs, "s_down", types[3], 2.0 ** -8)
+    base = rng.standard_normal(H).astype(np.float32)
+    base /= np.abs(base).max()
+    pos = [np.where(g > 0, g * u, 0.0) for g, u in gate_up(orc, spec, base)]   # silu(g) is g or 0 for a large g
+    top = max(np.abs(h).max() for h in pos)
+    X = np.stack([base * np.float32(np.sqrt(m / top)) for m in (1.0e37, 1.6e38, 2.9e38, 3.3e38)])
+    # a small route weight: y itself stays in range
+    desc.global_scale = spec["global_scale"] = 2.0 ** -12
+    y, idx, w = run(dev, desc, X)
+    for t in range(len(X)):
+        y_ref, logits, _, _ = orc.moe_layer(spec, X[t])
+        assert np.all(np.isfinite(y_ref)), "the reference overflows: scale the case down"
+        assert np.all(np.isfinite(y[t])), t
+        # silu(g) u: g and u are each within 2e-6 of the oracle's
+        err = np.abs(y[t].astype(np.float64) - y_ref).max()
+        assert err <= 2e-5 * np.abs(y_ref).max(), (t, err)
     for b in bufs.values():
         dev.free(b)
