@@ -4,15 +4,19 @@
 // Q6_K, Q8_0 shared) and for mixes of those with Q2_K, Q3_K and Q4_K.
 //
 // Activations (x per token for gate/up, h per pair for down) travel as "PH"
-// rows: per row a power-of-two scale s > max|v| (s = 1 for a zero row,
-// +inf when the row holds a NaN or an infinity, which then makes every
-// output of the row non-finite), and per column v' = v / s (|v'| < 1,
-// exact) as two f16 planes, hi = f16(v') and lo = f16(v' - hi): together
-// within 2^-23 of v' (lo's rounding, or the f16 subnormal spacing 2^-24).
+// rows: per row a power-of-two scale s with 2^15 s > max|v| (+inf when the
+// row holds a NaN or an infinity, which then makes every output of the row
+// non-finite), and per column v' = v / s (|v'| < 2^15, exact) as two f16
+// planes, hi = f16(v') and lo = f16(v' - hi): together within 2^-23 |v'| (two
+// roundings) or 2^-25 (lo's, among the f16 subnormals), which is at most
+// 2^-39 of the row's largest: beside an outlier 10^4 times the rest, the rest
+// keep their 22 bits (with |v'| < 1 the floor was 2^-24 of the outlier, and
+// outputs that it does not reach were 2.6e-3 off).
 // 128 columns of a row are a 576-byte record: hi (128 f16, column order),
 // lo (128 f16), then four 16-byte groups, one per 32 columns, for the min
-// terms of Q2_K, Q4_K and Q5_K: the two 16-column sums of v', each as three
-// f16 (together within 2^-25 of the f32 sum), and two zeros.
+// terms of Q2_K, Q4_K and Q5_K: the two 16-column sums of v', each / 16 (so
+// that it fits f16) as three f16 (together exact, or within 2^-25), and two
+// zeros.
 //
 // Weights enter v_mfma_f32_16x16x32_f16 as exact f16 integer codes, decoded
 // from the raw blocks in registers (the products hi * code and lo * code are
@@ -27,7 +31,7 @@
 //            (quants.c:203-226)
 //   Q4_K     code = q * sc, 6-bit sc per 32 (<= 15 * 63); sum w x = d C -
 //   Q5_K     dmin sum_j m_j S_j (Q5_K: code <= 31 * 63), the min terms as one
-//            more matrix op: the records' sums against the mins
+//            more matrix op: the records' sums against the mins, times 16
 //            (quants.c:104-151)
 //   Q2_K     the same with 4-bit sc and m per 16 weights (<= 3 * 15)
 //   Q3_K     code = (q - 4) * (sc - 32), sc per 16; sum w x = d C
@@ -134,14 +138,14 @@ extern "C" __global__ __launch_bounds__(256) void sepia_ph_quant(const float *__
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
     m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    // s = 2^e > m (exact scaling): e = the exponent of m's leading bit + 1,
-    // held to where s and 1 / s are both normal floats. 2^127 <= m: |v'| < 2,
-    // still exact in f16 hi + lo. m < 2^-126: every v is a multiple of 2^-149,
-    // every v' one of 2^-23, exact too.
+    // s = 2^e, 2^15 s > m (exact scaling): e = the exponent of m's leading
+    // bit + 1 - 15, held to where s is a normal float (1 / s is one then too).
+    // Where that holds it, m < 2^-111; rows below 2^-126 are multiples of
+    // 2^-149, whose v' are multiples of 2^-23, exact.
     const bool fin = m < INFINITY;
     int e = 0;
     if (fin && m > 0.0f) (void)frexpf(m, &e);
-    e = e < -126 ? -126 : e < 127 ? e : 127;
+    e = e - 15 < -126 ? -126 : e - 15;
     const float s = !fin ? INFINITY : ldexpf(1.0f, e), inv = fin ? ldexpf(1.0f, -e) : 0.0f;
     if (threadIdx.x == 0) scale[r] = s;
     uint8_t *out = rec + r * ldr;
@@ -167,7 +171,7 @@ extern "C" __global__ __launch_bounds__(256) void sepia_ph_quant(const float *__
             *(uint4 *)(blk + 32 * j + 16 * i) = *(const uint4 *)(h + 8 * i);
             *(uint4 *)(blk + 256 + 32 * j + 16 * i) = *(const uint4 *)(l + 8 * i);
         }
-        sum = fin ? sum : 0.0f;
+        sum = fin ? sum * 0.0625f : 0.0f;
         const _Float16 s0 = (_Float16)sum, s1 = (_Float16)(sum - (float)s0),
                        s2 = (_Float16)(sum - (float)s0 - (float)s1);
         _Float16 *sp = (_Float16 *)(blk + 512 + 16 * (j >> 1)) + 3 * (j & 1);
@@ -646,7 +650,7 @@ __device__ __forceinline__ void ph_proj(uint8_t *smem, const uint8_t *W0, const 
                         if constexpr (T == ST_Q6_K) c = __builtin_fmaf(16.0f, cb2[t][mt][k], c);
                         acc[t][mt][k] = __builtin_fmaf(d, c, acc[t][mt][k]);
                         if constexpr (F::MIN)
-                            acc[t][mt][k] = __builtin_fmaf(-ph_hhi(h[t][0]), cm[t][mt][k], acc[t][mt][k]);
+                            acc[t][mt][k] = __builtin_fmaf(-16.0f * ph_hhi(h[t][0]), cm[t][mt][k], acc[t][mt][k]);
                     }
             }
         }

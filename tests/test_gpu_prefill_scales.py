@@ -1,7 +1,8 @@
 """The f16 prefill path's row scales: rows whose largest magnitude is a
-denormal or close to the largest float. One routed and one shared expert, so
-that h of either follows from two of the oracle's matvecs; each token against
-the oracle's layer."""
+denormal or close to the largest float, and rows whose largest element the
+weights do not look at. One routed and one shared expert, so that h of either
+follows from two of the oracle's matvecs; each token against the oracle's
+layer."""
 import numpy as np
 import pytest
 
@@ -28,12 +29,14 @@ def layer(dev, rng, types):
     return desc, spec, bufs
 
 
-def rescale(dev, spec, bufs, name, t, factor):
-    """The f16 scales of a projection's blocks times a factor."""
-    blocks = spec[name][0].reshape(-1, synth.GEOM[t][1])
+def rescale(dev, spec, bufs, name, t, factor, columns=None):
+    """The f16 scales of a projection's blocks (those of the first columns of each row) times a factor."""
+    elems, nbytes = synth.GEOM[t]
+    blocks = spec[name][0].reshape(H, -1, nbytes)
+    n = blocks.shape[1] if columns is None else columns // elems
     for off in synth.F16_FIELDS[t]:
-        f = blocks[:, off:off + 2].copy().view(np.float16) * np.float16(factor)
-        blocks[:, off:off + 2] = f.view(np.uint8).reshape(-1, 2)
+        f = blocks[:, :n, off:off + 2].copy().view(np.float16) * np.float16(factor)
+        blocks[:, :n, off:off + 2] = f.view(np.uint8)
     dev.upload(bufs[name], spec[name][0])
 
 
@@ -103,5 +106,27 @@ def test_huge_rows(dev, orc, types):
         # silu(g) u: g and u are each within 2e-6 of the oracle's
         err = np.abs(y[t].astype(np.float64) - y_ref).max()
         assert err <= 2e-5 * np.abs(y_ref).max(), (t, err)
+    for b in bufs.values():
+        dev.free(b)
+
+
+@pytest.mark.parametrize("types", TYPES, ids=str)
+def test_outliers(dev, orc, types):
+    """One element of x many times the rest, in a block whose weights are zero: the other elements keep their
+    precision."""
+    rng = np.random.default_rng(sum(types) + 2)
+    desc, spec, bufs = layer(dev, rng, types)
+    for name in ("gate", "up", "s_gate", "s_up"):
+        rescale(dev, spec, bufs, name, spec["ts_gate" if name[1] == "_" else "t_gate"], 0.0, columns=256)
+    X = rng.standard_normal((4, H)).astype(np.float32)
+    X[1:, 77] = (1e3, -1e4, 1e5)
+    y, idx, w = run(dev, desc, X)
+    for t in range(len(X)):
+        y_ref, logits, _, _ = orc.moe_layer(spec, X[t])
+        check_route(orc, spec, logits, idx[t], w[t])
+        # an element's two planes hold it within 2^-23 of itself or 2^-39 of the row's largest (2e-7 here), the sums
+        # are f32: a few 2^-24 a contraction
+        err = np.abs(y[t].astype(np.float64) - y_ref).max()
+        assert err <= 4e-6 * np.abs(y_ref).max(), (t, err / np.abs(y_ref).max())
     for b in bufs.values():
         dev.free(b)
