@@ -281,6 +281,9 @@ struct AttnWave {
     }
     // Running maximum over the NC tiles' scores; sums so far rescaled where
     // it grew; the weights to LDS (ps: 16 rows of ATT_PS floats, the wave's own).
+    // A row whose scores so far are all -inf has that as its maximum and takes
+    // its weights against 0 (they are 0, and NaN for a NaN): a later score may
+    // be finite.
     template <int NC>
     __device__ __forceinline__ void weights(const att_f4 *s, int32_t c0, float *ps) {
         const int lane = (int)(threadIdx.x & 63), j = lane & 15, g = lane >> 4;
@@ -308,6 +311,9 @@ struct AttnWave {
                 m[r] = mn[r];
             }
         }
+        float mb[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) mb[r] = m[r] == -INFINITY ? 0.0f : m[r];
 #pragma unroll
         for (int c = 0; c < NC; c++) {
             __builtin_amdgcn_sched_barrier(0);
@@ -316,7 +322,7 @@ struct AttnWave {
                 const int32_t kv = c0 + 16 * c + j;
                 const uint32_t in = kv >= lo[r] && kv <= hi[r] ? 0xFFFFFFFFu : 0u;
                 const float p = __builtin_bit_cast(
-                    float, __builtin_bit_cast(uint32_t, (float)att_exp(s[c][r] - m[r])) & in);
+                    float, __builtin_bit_cast(uint32_t, (float)att_exp(s[c][r] - mb[r])) & in);
                 l[r] += (double)p;
                 ps[(4 * g + r) * ATT_PS + 16 * c + j] = p;
             }

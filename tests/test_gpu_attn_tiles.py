@@ -81,3 +81,20 @@ def test_nonfinite_rows(dev, orc, bad, T, H, Hkv, n, window):
     args[1][(n - 1) * args[13] + 3] = bad
     args[1][max(0, args[4][0] - 1) * args[13]] = bad
     check(dev, orc, args)
+
+
+@pytest.mark.parametrize("low", [-np.inf, float(np.finfo(np.float32).min)], ids=["-inf", "lowest"])
+@pytest.mark.parametrize("T,H,Hkv,n,window", [(1, 8, 1, 20, 20), (1, 64, 8, 4097, 4097), (2, 16, 2, 60, 40),
+                                              (40, 8, 4, 200, 64), (70, 8, 2, 150, 150)], ids=str)
+def test_masked_scores(dev, orc, low, T, H, Hkv, n, window):
+    """A band bias of -inf or the lowest float takes whole steps, waves and splits out of a row, at its start, at its
+    end, everywhere but one position or everywhere: the reference's maximum is over the whole row, so a row gives NaN
+    only where every score is -inf."""
+    args = make(np.random.default_rng(T + n), T, H, Hkv, 128, n, n, window)
+    rel = args[3].reshape(T, H, n)   # by distance from the token
+    rel[:, 0, min(window, n) // 2:] = low
+    rel[:, 1, :min(window, n) // 2 + 1] = low
+    rel[:, 2, :] = low
+    rel[:, 2, min(5, T - 1):1 + min(5, T - 1)] = 0.25
+    rel[T - 1, 3, :] = low
+    check(dev, orc, args)
