@@ -1283,9 +1283,11 @@ static size_t scratch_limit(void) {
     return g_scratch ? g_scratch_len - CNT_BYTES : 0;
 }
 
-/* Tokens t0 .. t0 + T - 1 (T <= ATT_TMAX) of a call whose arguments are checked. */
+/* Tokens t0 .. t0 + T - 1 (T <= ATT_TMAX) of a call whose arguments are
+ * checked. fold: through partials and the fold launch even without a split
+ * (the outputs lie in an input that other workgroups read). */
 static int attn_launch(const char *op, AttnArgs a, int64_t t0, const int64_t *kv_lo, const int64_t *kv_hi,
-                       const float *tau) {
+                       const float *tau, int fold) {
     const int64_t T = a.T, G = a.H / a.Hkv;
     /* Few rows: the waves of a workgroup split the kv range of 16 rows and
      * read k and v once each from global memory. Many: 64 rows share the k
@@ -1319,11 +1321,12 @@ static int attn_launch(const char *op, AttnArgs a, int64_t t0, const int64_t *kv
     a.span = span > 0x7FFFFFFF ? 0x7FFFFFFF : (int32_t)span;
     a.gtok = NULL;
     a.part = NULL;
-    if (bounds || nsplit > 1) {
-        uint8_t *s = (uint8_t *)scratch(bounds + (nsplit > 1 ? (size_t)nsplit * per : 0), op);
+    fold = fold || nsplit > 1;
+    if (bounds || fold) {
+        uint8_t *s = (uint8_t *)scratch(bounds + (fold ? (size_t)nsplit * per : 0), op);
         if (!s) return 0;
         if (bounds) a.gtok = (const int32_t *)s;
-        if (nsplit > 1) a.part = (double *)(s + bounds);
+        if (fold) a.part = (double *)(s + bounds);
     }
     AttnTok tok;
     memset(&tok, 0, sizeof tok);
@@ -1350,7 +1353,7 @@ static int attn_launch(const char *op, AttnArgs a, int64_t t0, const int64_t *kv
     const int kern = a.Dh == 128 ? (wave ? K_ATTN_WAVE : K_ATTN_TILE) : (wave ? K_ATTN_WAVE_D : K_ATTN_TILE_D);
     if (!launch3(kern, (unsigned)a.Hkv, (unsigned)tiles, (unsigned)nsplit, 256, 0, a_p, op))
         return 0;
-    if (nsplit == 1) return 1;
+    if (!fold) return 1;
     void *a_c[] = { &a.part, &a.H, &a.Dh, &a.nsplit, &a.out };
     return launch2(K_ATTN_COMBINE, (unsigned)a.H, (unsigned)T, 128, 0, a_c, op);
 }
@@ -1410,7 +1413,9 @@ int sepia_gpu_banded_attn(SepiaGpuBuf *q, SepiaGpuBuf *k, SepiaGpuBuf *v, SepiaG
         a.Dh = (int32_t)Dh;
         a.R = (int32_t)rel_extent;
         a.inv_head_dim = inv_head_dim;
-        if (!attn_launch(op, a, t0, kv_lo, kv_hi, tau)) return 0;
+        /* a workgroup reads the q of its own outputs only, and before it writes */
+        const int fold = attn_out->dev == k->dev || attn_out->dev == v->dev || attn_out->dev == rel_logits->dev;
+        if (!attn_launch(op, a, t0, kv_lo, kv_hi, tau, fold)) return 0;
     }
     return 1;
 }

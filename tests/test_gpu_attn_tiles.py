@@ -5,6 +5,8 @@ the bounds in the kernel arguments (64, then 256 a launch), kv ranges off the
 16- and 32-row steps and split over workgroups, and NaN or infinite v rows
 that only some of a tile's rows see. All against the oracle's restatement of
 the reference's loop (src/sepia.c:1203-1247)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -98,3 +100,23 @@ def test_masked_scores(dev, orc, low, T, H, Hkv, n, window):
     rel[:, 2, min(5, T - 1):1 + min(5, T - 1)] = 0.25
     rel[T - 1, 3, :] = low
     check(dev, orc, args)
+
+
+@pytest.mark.parametrize("T,H,Hkv,n", [(1, 8, 1, 20), (3, 16, 2, 70), (60, 4, 2, 200)], ids=str)
+@pytest.mark.parametrize("shared", ["q", "k", "v", "rel_logits"])
+def test_output_in_an_input(dev, orc, shared, T, H, Hkv, n):
+    """attn_out may be one of the inputs: every input is read before the first output is written (q, which a
+    workgroup reads for its own outputs only, in any case)."""
+    args = make(np.random.default_rng(T + n), T, H, Hkv, 128, 128, n, n)
+    q, k, v, rl, lo, hi, tau, _, _, _, Dh, R, qpb, kv_dim = args
+    names = ["q", "k", "v", "rel_logits"]
+    bufs = [dev.shared_from(a) for a in (q, k, v, rl)]
+    out = bufs[names.index(shared)]
+    c = [ctypes.cast(a, ctypes.c_void_p) for a in ((ctypes.c_int64 * T)(*lo), (ctypes.c_int64 * T)(*hi),
+                                                   (ctypes.c_float * T)(*tau))]
+    dev.run(dev.L.sepia_gpu_banded_attn, *bufs, out, *c, T, H, Hkv, Dh, R, qpb, kv_dim, 1.0 / Dh)
+    got = dev.download(out, T * H * Dh)
+    want = orc.banded_attn(*args, 1.0 / Dh)
+    assert np.abs(got.astype(np.float64) - want).max() <= 5e-6 * np.abs(want).max()
+    for b in bufs:
+        dev.free(b)
