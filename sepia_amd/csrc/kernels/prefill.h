@@ -389,15 +389,17 @@ __device__ __forceinline__ void pf_issue_act(const __bf16 *src_hi, const __bf16 
 
 // Raw blocks b of nr rows (rows r0 .. r0 + nr - 1 of a matrix of `rows`
 // rows; rows past the end repeat the last one) into dst, row k at k * 4 RD:
-// each row's 4-byte-aligned window that holds the block.
+// each row's 4-byte-aligned window that holds the block (32-bit offsets from
+// row r0, so that they reach its rows in a matrix of any size).
 template <int T>
 __device__ __forceinline__ void pf_issue_raw(const uint8_t *W, uint64_t row_bytes, int64_t rows, int64_t r0, int nr,
                                              int64_t b, uint8_t *dst) {
     constexpr int BB = Fmt<T>::bytes, RD = (BB + 6) / 4;
     const int nw = (int)(blockDim.x >> 6), w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
-    const uint8_t *Wa = (const uint8_t *)((uintptr_t)W & ~(uintptr_t)3);
-    const uint32_t delta = (uint32_t)((uintptr_t)W & 3);
+    const uint8_t *W0 = W + (uint64_t)r0 * row_bytes;
+    const uint8_t *Wa = (const uint8_t *)((uintptr_t)W0 & ~(uintptr_t)3);
+    const uint32_t delta = (uint32_t)((uintptr_t)W0 & 3);
     const int n_ins = (nr * RD + 63) >> 6;
     for (int j = w; j < n_ins; j += nw) {
         const int i = 64 * j + lane;
@@ -405,7 +407,7 @@ __device__ __forceinline__ void pf_issue_raw(const uint8_t *W, uint64_t row_byte
             const int r = i / RD, d = i - r * RD;
             int64_t rr = r0 + r;
             rr = rr < rows ? rr : rows - 1;
-            const uint64_t off = delta + (uint64_t)rr * row_bytes + (uint64_t)b * BB;
+            const uint64_t off = delta + (uint64_t)(rr - r0) * row_bytes + (uint64_t)b * BB;
             pf_dma4(Wa, (uint32_t)(off & ~(uint64_t)3) + 4u * (uint32_t)d, pf_lds(dst + 256 * j));
         }
     }

@@ -511,10 +511,12 @@ __device__ __forceinline__ void ph_proj(uint8_t *smem, const uint8_t *W0, const 
 #pragma unroll
     for (int k = 0; k < KW; k++) {
         const int q = 64 * k + l < 16 * PW ? 64 * k + l : 0, m = q / PW;
-        wrow[k] = on ? (uint32_t)((uint64_t)(grow + m) * row_bytes) : 0u;
+        wrow[k] = (uint32_t)((uint64_t)m * row_bytes);
         wcol[k] = 16u * (uint32_t)(q - m * PW);
     }
-    const uint8_t *Wt[NT] = {W0, GU ? W1 : W0 + (on ? 16 * row_bytes : 0)};
+    // (from the wave's first row: 32-bit offsets then reach its rows in a matrix of any size)
+    const uint64_t wfirst = on ? (uint64_t)grow * row_bytes : 0;
+    const uint8_t *Wt[NT] = {W0 + wfirst, GU ? W1 + wfirst : W0 + wfirst + (on ? 16 * row_bytes : 0)};
     uint8_t *wl = smem + O_W + (uint32_t)w * (NT * 16 * 16 * PW);
     ph_u4 wr[NT][KW];
     auto w_load = [&](int b) {   // the group of blocks b ..

@@ -159,9 +159,8 @@ struct PqDma {
     static_assert(NW % 8 == 0 && 64 * KW == 32 * PW, "a wave stages its own 32 rows");
     static_assert(PF_MT * AP % 64 == 0, "a record stage is whole DMA instructions");
     uint32_t a[KA];            // record piece offsets at block 0
-    uint32_t r[KW], c16[KW];   // row offset from the matrix base; offset of the lane's piece
-    __device__ __forceinline__ void init(const uint32_t *roff, const uint8_t *W0, const uint8_t *W1,
-                                         uint64_t row_bytes, int64_t r0) {
+    uint32_t r[KW], c16[KW];   // row offset from the workgroup's first row; offset of the lane's piece
+    __device__ __forceinline__ void init(const uint32_t *roff, uint64_t row_bytes) {
         const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
 #pragma unroll
         for (int k = 0; k < KA; k++) {
@@ -173,7 +172,7 @@ struct PqDma {
             const int jj = KW * w + k;
             const int mat = GU ? jj / (NW / 2) : 0, j1 = GU ? jj - mat * (NW / 2) : jj;
             const int q = 64 * j1 + lane, kr = q / PW, c = q - kr * PW;
-            r[k] = (uint32_t)((uint64_t)(r0 + kr) * row_bytes);
+            r[k] = (uint32_t)((uint64_t)kr * row_bytes);
             c16[k] = 16 * c >= BB ? 0u : 16 * c + 16 <= BB + 2 ? 16u * (uint32_t)c : (uint32_t)(BB - 16);
         }
     }
@@ -561,8 +560,9 @@ __device__ __forceinline__ void pq_wait_vm(int n) {
 
 // One projection workgroup (see the top of the file). GU: rows r0 .. r0 +
 // 127 of gate (W0) and up (W1), h[pair][row] = silu(gate) * up in f32;
-// down: rows r0 .. r0 + 255 of W0, out[pair][row] in f32. ld_out: floats
-// per output row (I for h, H for the down partials).
+// down: rows r0 .. r0 + 255 of W0, out[pair][row] in f32 (W0, W1: row r0 of
+// either, so that 32-bit offsets reach a workgroup's rows in a matrix of any
+// size). ld_out: floats per output row (I for h, H for the down partials).
 template <int T, bool GU, int MT>
 __device__ __forceinline__ void pq_proj(uint8_t *smem, const uint8_t *W0, const uint8_t *W1, uint64_t row_bytes,
                                         int64_t nb, const uint8_t *pq, const uint32_t *roff, const int32_t *pair,
@@ -578,7 +578,7 @@ __device__ __forceinline__ void pq_proj(uint8_t *smem, const uint8_t *W0, const 
     auto a_stage = [&](int b) { return smem + (uint32_t)(b & 1) * a_bytes; };
     auto w_stage = [&](int b) { return smem + 2 * a_bytes + (uint32_t)b % SW * w_bytes; };
     PqDma<T, GU> dma;
-    dma.init(roff, W0, W1, row_bytes, r0);
+    dma.init(roff, row_bytes);
     const int nwi = PqDma<T, GU>::n_w();
     pf_f32x4 acc[2][2];
 #pragma unroll
@@ -710,8 +710,8 @@ extern "C" __global__ __launch_bounds__(512) void sepia_pf_gateup_q(
     const bool routed = e < n_routed;
     const PfProj &G = routed ? gate : s_gate, &U = routed ? up : s_up;
     const int64_t ei = routed ? e : e - n_routed;
-    const uint8_t *wg = G.base + ei * G.stride, *wu = U.base + ei * U.stride;
     const int64_t r0 = (int64_t)blockIdx.x * 128;
+    const uint8_t *wg = G.base + ei * G.stride + r0 * G.row_bytes, *wu = U.base + ei * U.stride + r0 * G.row_bytes;
     uint32_t *roff;
     int32_t *pair;
     float *srow;
@@ -734,8 +734,8 @@ extern "C" __global__ __launch_bounds__(512) void sepia_pf_down_q(
     const bool routed = e < n_routed;
     const PfProj &D = routed ? down : s_down;
     const int64_t ei = routed ? e : e - n_routed;
-    const uint8_t *wd = D.base + ei * D.stride;
     const int64_t r0 = (int64_t)blockIdx.x * 256;
+    const uint8_t *wd = D.base + ei * D.stride + r0 * D.row_bytes;
     uint32_t *roff;
     int32_t *pair;
     float *srow;

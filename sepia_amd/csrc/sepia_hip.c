@@ -2215,14 +2215,11 @@ int sepia_gpu_moe_prefill(const SepiaMoeLayerDesc *L, int64_t n_tokens, SepiaGpu
      * with the int8 ones (moe_prefill of a Q4_K / Q6_K layer at hidden 4096,
      * 300 tokens: 1.82 ms on the bf16 kernels, 0.59 ms here), rows 4-byte
      * aligned; the bf16 kernels take what is left: layers with rows at 2-byte
-     * offsets, and mixes whose activation records pass the bound below, with
-     * a matrix that the f16 kernels' 32-bit row offsets do not span, or whose
-     * scratch (more than the bf16 path's) a capture does not hold */
-    int use_h = !use_q && g_opt_pf_h && q_aligned, span = 1;
-    for (int i = 0; i < (ns > 0 ? 6 : 3); i++)
-        if ((uint64_t)(i % 3 == 2 ? H : I) * ps[i]->row_bytes >= (1ull << 32)) span = 0;
+     * offsets, and mixes whose activation records pass the bound below or
+     * whose scratch (more than the bf16 path's) a capture does not hold */
+    int use_h = !use_q && g_opt_pf_h && q_aligned;
     if (use_h && !use_h_all &&
-        (!span || pf_rows_large(T, H, PF_HREC) || pf_rows_large(P, I, PF_HREC) ||
+        (pf_rows_large(T, H, PF_HREC) || pf_rows_large(P, I, PF_HREC) ||
          pf_scratch(T, H, I, n_tot, tk, n_sel, pf_units(T, tk, nr, ns, PH_UM), PH_REC * 2).bytes > scratch_limit()))
         use_h = 0;
     const int use_qh = use_q || use_h;
