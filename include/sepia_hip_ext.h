@@ -83,8 +83,11 @@ int sepia_hip_moe_decode_noalloc(const SepiaMoeLayerDesc *layer, SepiaGpuBuf *x,
  * activations as f16 hi + lo planes), all with f32 accumulation. Rows 4-byte
  * aligned; layers with rows at 2-byte offsets (without Q8_0) run on the bf16
  * ones (weights and activations as bf16 hi + lo pairs), and so do layers of
- * both kinds whose f16 scratch a capture does not hold. x, y: f32
- * [n_tokens][hidden] at offset 0.
+ * both kinds from n_tokens * hidden or n_tokens * slots * inter of about
+ * 1.04e9 on. While the stream is being captured, a call whose scratch holds
+ * the bf16 kernels' needs but not the f16 ones' runs on the latter in parts of
+ * the tokens, with the same bits (one or two tokens whose part does not fit:
+ * on the bf16 ones, without Q8_0). x, y: f32 [n_tokens][hidden] at offset 0.
  * route_out (optional): int32 idx[n_tokens][topk] followed by f32
  * w[n_tokens][topk + n_shared]. */
 int sepia_gpu_moe_prefill(const SepiaMoeLayerDesc *layer, int64_t n_tokens, SepiaGpuBuf *x, SepiaGpuBuf *y,

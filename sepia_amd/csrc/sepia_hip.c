@@ -2112,29 +2112,30 @@ static int pf_rows_large(int64_t rows, int64_t n, int64_t rec) {
  * 64-bit offsets, so its larger records may pass it) */
 #define PF_HREC 1056
 
-/* Regions of a call's scratch; rec: bytes of a 256-column record of the int8
- * or f16 path, 0 for the bf16 path. */
+/* Regions of a call's scratch: the routing of all T tokens, the rest for
+ * parts of n tokens. rec: bytes of a 256-column record of the int8 or f16
+ * path, 0 for the bf16 path; um: pairs per unit. */
 typedef struct {
     size_t logits, idx, w, list, units, nu, xh, xl, hh, hl, pqx, pqxs, pqh, pqhs, yp, bytes;
 } PfScratch;
-static PfScratch pf_scratch(int64_t T, int64_t H, int64_t I, int64_t n_tot, int64_t tk, int64_t n_sel, int64_t umax,
-                            int64_t rec) {
-    const int64_t P = T * n_sel;
+static PfScratch pf_scratch(int64_t T, int64_t n, int64_t H, int64_t I, int64_t nr, int64_t ns, int64_t tk,
+                            int64_t um, int64_t rec) {
+    const int64_t P = n * (tk + ns);
     PfScratch o;
     memset(&o, 0, sizeof o);
-#define PF_REGION(name, n) o.name = o.bytes, o.bytes += ((size_t)(n) + 255) & ~(size_t)255
-    PF_REGION(logits, T * n_tot * 4);
+#define PF_REGION(name, len) o.name = o.bytes, o.bytes += ((size_t)(len) + 255) & ~(size_t)255
+    PF_REGION(logits, T * (nr + ns) * 4);
     PF_REGION(idx, T * tk * 4);
-    PF_REGION(w, P * 4);
+    PF_REGION(w, T * (tk + ns) * 4);
     PF_REGION(list, P * 4);
-    PF_REGION(units, umax * 12);
+    PF_REGION(units, pf_units(n, tk, nr, ns, um) * 12);
     PF_REGION(nu, 4);   /* n_units */
-    PF_REGION(xh, rec ? 0 : T * H * 2);
-    PF_REGION(xl, rec ? 0 : T * H * 2);
+    PF_REGION(xh, rec ? 0 : n * H * 2);
+    PF_REGION(xl, rec ? 0 : n * H * 2);
     PF_REGION(hh, rec ? 0 : P * I * 2);
     PF_REGION(hl, rec ? 0 : P * I * 2);
-    PF_REGION(pqx, T * (H / 256 * rec));
-    PF_REGION(pqxs, rec ? T * 4 : 0);
+    PF_REGION(pqx, n * (H / 256 * rec));
+    PF_REGION(pqxs, rec ? n * 4 : 0);
     PF_REGION(pqh, P * (I / 256 * rec));
     PF_REGION(pqhs, rec ? P * 4 : 0);
     /* the down launch's partial rows take the place of h in f32, which is
@@ -2215,16 +2216,31 @@ int sepia_gpu_moe_prefill(const SepiaMoeLayerDesc *L, int64_t n_tokens, SepiaGpu
      * with the int8 ones (moe_prefill of a Q4_K / Q6_K layer at hidden 4096,
      * 300 tokens: 1.82 ms on the bf16 kernels, 0.59 ms here), rows 4-byte
      * aligned; the bf16 kernels take what is left: layers with rows at 2-byte
-     * offsets, and mixes whose activation records pass the bound below or
-     * whose scratch (more than the bf16 path's) a capture does not hold */
+     * offsets, and mixes whose activation records pass the bound below */
     int use_h = !use_q && g_opt_pf_h && q_aligned;
-    if (use_h && !use_h_all &&
-        (pf_rows_large(T, H, PF_HREC) || pf_rows_large(P, I, PF_HREC) ||
-         pf_scratch(T, H, I, n_tot, tk, n_sel, pf_units(T, tk, nr, ns, PH_UM), PH_REC * 2).bytes > scratch_limit()))
-        use_h = 0;
+    if (use_h && !use_h_all && (pf_rows_large(T, H, PF_HREC) || pf_rows_large(P, I, PF_HREC))) use_h = 0;
+    /* A capture whose scratch holds the bf16 path's regions, but not the f16
+     * path's (up to 2.2 times those), is taken in the fewest even parts of the
+     * tokens that fit: the same routing and the same sums, so the same bits as
+     * without a capture. Only where a single token's part does not fit (one
+     * or two tokens on very long rows) the bf16 kernels run. */
+    int64_t part = T;
+    if (use_h) {
+        const size_t limit = scratch_limit();
+        if (pf_scratch(T, T, H, I, nr, ns, tk, 32, 0).bytes <= limit) {
+            for (int64_t n = 2; pf_scratch(T, part, H, I, nr, ns, tk, PH_UM, PH_REC * 2).bytes > limit && part > 1; n++)
+                part = (T + n - 1) / n;
+            int q8 = 0;
+            for (int i = 0; i < (ns > 0 ? 6 : 3); i++) q8 |= ps[i]->type == 8;
+            if (pf_scratch(T, part, H, I, nr, ns, tk, PH_UM, PH_REC * 2).bytes > limit && !q8) {
+                use_h = 0;
+                part = T;
+            }
+        }
+    }
     const int use_qh = use_q || use_h;
     const int64_t rec = use_h ? PH_REC * 2 : 832, ldqx = H / 256 * rec, ldqh = I / 256 * rec;
-    const int64_t um = use_h ? PH_UM : 32, umax = pf_units(T, tk, nr, ns, um);
+    const int64_t um = use_h ? PH_UM : 32, umax = pf_units(part, tk, nr, ns, um);
     /* grid rows of the f16 unit kernels: a multiple of 8, so they deal the
      * units to the 8 XCDs in turn (kernels/prefill.h pf_slot) */
     const int64_t ugrid = (umax + 7) & ~(int64_t)7;
@@ -2238,7 +2254,7 @@ int sepia_gpu_moe_prefill(const SepiaMoeLayerDesc *L, int64_t n_tokens, SepiaGpu
     }
     if (!need_batch(op)) return 0;
 
-    const PfScratch o = pf_scratch(T, H, I, n_tot, tk, n_sel, umax, use_qh ? rec : 0);
+    const PfScratch o = pf_scratch(T, part, H, I, nr, ns, tk, um, use_qh ? rec : 0);
     uint8_t *s = (uint8_t *)scratch(o.bytes, op);
     if (!s) return 0;
     float *logits = (float *)(s + o.logits), *sel_w = (float *)(s + o.w), *yp = (float *)(s + o.yp);
@@ -2267,45 +2283,51 @@ int sepia_gpu_moe_prefill(const SepiaMoeLayerDesc *L, int64_t n_tokens, SepiaGpu
     void *a_sel[] = { &logits, &rb, &nr32, &ns32, &tk32, &rs, &gsc, &sel_idx, &sel_w };
     if (!launch(K_PF_SELECT, (unsigned)T, 64, a_sel, op)) return 0;
     int32_t um32 = (int32_t)um;
-    void *a_grp[] = { &sel_idx, &tt, &nr32, &ns32, &tk32, &um32, &list, &units, &n_units };
-    if (!launch(K_PF_GROUP, 1, 1024, a_grp, op)) return 0;
-    if (use_qh) {
-        /* int8 (PQ rows) or f16 (PH rows): quantize x, gate/up to f32 h,
-         * quantize h, down to the per-pair partial rows. Gate/up runs over
-         * 128-row slices of I, down over 256-row slices of H. */
-        void *pqx = s + o.pqx, *pqxs = s + o.pqxs, *hf = s + o.yp, *pqh = s + o.pqh, *pqhs = s + o.pqhs;
-        int64_t ldq_x = ldqx, ldq_h = ldqh;
-        const int kq = use_q ? K_PF_QUANT : K_PH_QUANT;
-        void *a_qx[] = { &x->dev, &hid, &hid, &pqx, &ldq_x, &pqxs };
-        if (!launch(kq, (unsigned)T, 256, a_qx, op)) return 0;
-        void *a_qh[] = { &hf, &inter, &inter, &pqh, &ldq_h, &pqhs };
-        if (use_q) {
-            void *a_gq[] = { (void *)&g, (void *)&u, (void *)&sg, (void *)&su, &nr32, &nsel32, &inter, &hid,
-                             &pqx, &pqxs, &list, &units, &n_units, &hf };
-            if (!launch2(K_PF_GATEUP_Q, (unsigned)(I / 128), (unsigned)umax, 512, PF_LDS_BYTES, a_gq, op)) return 0;
-            if (!launch(kq, (unsigned)P, 256, a_qh, op)) return 0;
-            void *a_dq[] = { (void *)&d, (void *)&sd, &nr32, &inter, &hid, &pqh, &pqhs, &list, &units, &n_units, &yp };
-            if (!launch2(K_PF_DOWN_Q, (unsigned)(H / 256), (unsigned)umax, 512, PF_LDS_BYTES, a_dq, op)) return 0;
+    for (int64_t t0 = 0; t0 < T; t0 += part) {
+        int64_t n = T - t0 < part ? T - t0 : part;
+        const float *xd = (const float *)x->dev + t0 * H, *wt = sel_w + t0 * n_sel;
+        const int32_t *it = sel_idx + t0 * tk;
+        float *yd = (float *)y->dev + t0 * H;
+        void *a_grp[] = { &it, &n, &nr32, &ns32, &tk32, &um32, &list, &units, &n_units };
+        if (!launch(K_PF_GROUP, 1, 1024, a_grp, op)) return 0;
+        if (use_qh) {
+            /* int8 (PQ rows) or f16 (PH rows): quantize x, gate/up to f32 h,
+             * quantize h, down to the per-pair partial rows. Gate/up runs over
+             * 128-row slices of I, down over 256-row slices of H. */
+            void *pqx = s + o.pqx, *pqxs = s + o.pqxs, *hf = s + o.yp, *pqh = s + o.pqh, *pqhs = s + o.pqhs;
+            int64_t ldq_x = ldqx, ldq_h = ldqh;
+            const int kq = use_q ? K_PF_QUANT : K_PH_QUANT;
+            void *a_qx[] = { &xd, &hid, &hid, &pqx, &ldq_x, &pqxs };
+            if (!launch(kq, (unsigned)n, 256, a_qx, op)) return 0;
+            void *a_qh[] = { &hf, &inter, &inter, &pqh, &ldq_h, &pqhs };
+            if (use_q) {
+                void *a_gq[] = { (void *)&g, (void *)&u, (void *)&sg, (void *)&su, &nr32, &nsel32, &inter, &hid,
+                                 &pqx, &pqxs, &list, &units, &n_units, &hf };
+                if (!launch2(K_PF_GATEUP_Q, (unsigned)(I / 128), (unsigned)umax, 512, PF_LDS_BYTES, a_gq, op)) return 0;
+                if (!launch(kq, (unsigned)(n * n_sel), 256, a_qh, op)) return 0;
+                void *a_dq[] = { (void *)&d, (void *)&sd, &nr32, &inter, &hid, &pqh, &pqhs, &list, &units, &n_units, &yp };
+                if (!launch2(K_PF_DOWN_Q, (unsigned)(H / 256), (unsigned)umax, 512, PF_LDS_BYTES, a_dq, op)) return 0;
+            } else {
+                void *a_gu[] = { (void *)&g, (void *)&u, (void *)&sg, (void *)&su, &nr32, &nsel32, &inter, &hid,
+                                 &pqx, &pqxs, &list, &units, &n_units, &hf };
+                if (!launch2(K_PH_GATEUP, (unsigned)(I / 128), (unsigned)ugrid, PH_THREADS, PH_LDS_BYTES, a_gu, op)) return 0;
+                if (!launch(kq, (unsigned)(n * n_sel), 256, a_qh, op)) return 0;
+                void *a_dn[] = { (void *)&d, (void *)&sd, &nr32, &inter, &hid, &pqh, &pqhs, &list, &units, &n_units, &yp };
+                if (!launch2(K_PH_DOWN, (unsigned)(H / 256), (unsigned)ugrid, PH_THREADS, PH_LDS_BYTES, a_dn, op)) return 0;
+            }
         } else {
-            void *a_gu[] = { (void *)&g, (void *)&u, (void *)&sg, (void *)&su, &nr32, &nsel32, &inter, &hid,
-                             &pqx, &pqxs, &list, &units, &n_units, &hf };
-            if (!launch2(K_PH_GATEUP, (unsigned)(I / 128), (unsigned)ugrid, PH_THREADS, PH_LDS_BYTES, a_gu, op)) return 0;
-            if (!launch(kq, (unsigned)P, 256, a_qh, op)) return 0;
-            void *a_dn[] = { (void *)&d, (void *)&sd, &nr32, &inter, &hid, &pqh, &pqhs, &list, &units, &n_units, &yp };
-            if (!launch2(K_PH_DOWN, (unsigned)(H / 256), (unsigned)ugrid, PH_THREADS, PH_LDS_BYTES, a_dn, op)) return 0;
+            int64_t nseg = n * H / 16;
+            void *a_sp[] = { &xd, &nseg, &xh, &xl };
+            if (!launch(K_PF_SPLIT, (unsigned)((nseg + 255) / 256), 256, a_sp, op)) return 0;
+            void *a_gu[] = { (void *)&g, (void *)&u, (void *)&sg, (void *)&su, &nr32, &nsel32, &inter, &hid, &xh, &xl,
+                             &list, &units, &n_units, &hh, &hl };
+            if (!launch2(K_PF_GATEUP, (unsigned)((I + 31) / 32), (unsigned)umax, 512, PF_LDS_BYTES, a_gu, op)) return 0;
+            void *a_dn[] = { (void *)&d, (void *)&sd, &nr32, &inter, &hid, &hh, &hl, &list, &units, &n_units, &yp };
+            if (!launch2(K_PF_DOWN, (unsigned)((H + 63) / 64), (unsigned)umax, 512, PF_LDS_BYTES, a_dn, op)) return 0;
         }
-    } else {
-        int64_t nseg = T * H / 16;
-        void *a_sp[] = { &x->dev, &nseg, &xh, &xl };
-        if (!launch(K_PF_SPLIT, (unsigned)((nseg + 255) / 256), 256, a_sp, op)) return 0;
-        void *a_gu[] = { (void *)&g, (void *)&u, (void *)&sg, (void *)&su, &nr32, &nsel32, &inter, &hid, &xh, &xl,
-                         &list, &units, &n_units, &hh, &hl };
-        if (!launch2(K_PF_GATEUP, (unsigned)((I + 31) / 32), (unsigned)umax, 512, PF_LDS_BYTES, a_gu, op)) return 0;
-        void *a_dn[] = { (void *)&d, (void *)&sd, &nr32, &inter, &hid, &hh, &hl, &list, &units, &n_units, &yp };
-        if (!launch2(K_PF_DOWN, (unsigned)((H + 63) / 64), (unsigned)umax, 512, PF_LDS_BYTES, a_dn, op)) return 0;
+        void *a_cb[] = { &yp, &wt, &nsel32, &n, &hid, &yd };
+        if (!launch2(K_PF_COMBINE, (unsigned)((H + 255) / 256), (unsigned)n, 256, 0, a_cb, op)) return 0;
     }
-    void *a_cb[] = { &yp, &sel_w, &nsel32, &tt, &hid, &y->dev };
-    if (!launch2(K_PF_COMBINE, (unsigned)((H + 255) / 256), (unsigned)T, 256, 0, a_cb, op)) return 0;
     if (route_out) {
         hipError_t e = hipMemcpyAsync(route_out->dev, sel_idx, (size_t)T * tk * 4, hipMemcpyDeviceToDevice, g_stream);
         if (e == hipSuccess)
