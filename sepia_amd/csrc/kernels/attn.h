@@ -145,26 +145,30 @@ __device__ __forceinline__ float att_max16(float v) {
     return v;
 }
 
-// e^x for x <= 0 (or NaN) to about 1e-11 relative in double, far below the
-// f32 rounding of the weights: x = n ln 2 + r, |r| <= ln 2 / 2, the Taylor
-// series of e^r to degree 9 (remainder r^10 / 10! < 7e-12) and an exact
-// scaling by 2^n. Below -200 (an f32 zero since -104) n stops growing. The
-// rounding to n adds 1.5 * 2^52, which leaves n in the sum's low word.
+// e^x for x <= 0 (or NaN) in double, within about 2^-51 of it: x = n ln 2 + r,
+// |r| <= ln 2 / 2 (ln 2 as the sum of two doubles), e^r as 1 + r q(r) with q
+// of degree 9 for the least largest relative error (Remez exchange; 2.3e-16 as
+// rounded here) and an exact scaling by 2^n. Below -200 (an f32 zero since
+// -104) n stops growing. The rounding to n adds 1.5 * 2^52, which leaves n in
+// the sum's low word. Two fused multiply-adds fewer (a Taylor series to degree
+// 9 and one ln 2) were 7e-12 off.
 __device__ __forceinline__ double att_exp(float x) {
     const double xd = (double)(x < -200.0f ? -200.0f : x);
     const double big = 6755399441055744.0;
     const double t = __builtin_fma(xd, 1.4426950408889634074, big);
     const int n = (int)(uint32_t)__builtin_bit_cast(uint64_t, t);
-    const double r = __builtin_fma(t - big, -0.69314718055994530942, xd);
-    double p = 1.0 / 362880.0;
-    p = __builtin_fma(p, r, 1.0 / 40320.0);
-    p = __builtin_fma(p, r, 1.0 / 5040.0);
-    p = __builtin_fma(p, r, 1.0 / 720.0);
-    p = __builtin_fma(p, r, 1.0 / 120.0);
-    p = __builtin_fma(p, r, 1.0 / 24.0);
-    p = __builtin_fma(p, r, 1.0 / 6.0);
-    p = __builtin_fma(p, r, 0.5);
-    p = __builtin_fma(p, r, 1.0);
+    const double nd = t - big;
+    const double r = __builtin_fma(nd, -2.3190468138462996e-17, __builtin_fma(nd, -0.69314718055994530942, xd));
+    double p = 0x1.27315c7a1d3bep-22;
+    p = __builtin_fma(p, r, 0x1.72f785aa9806cp-19);
+    p = __builtin_fma(p, r, 0x1.a01b59c924b4cp-16);
+    p = __builtin_fma(p, r, 0x1.a0197ca67eee6p-13);
+    p = __builtin_fma(p, r, 0x1.6c16c0cdd2530p-10);
+    p = __builtin_fma(p, r, 0x1.1111112c56a8dp-7);
+    p = __builtin_fma(p, r, 0x1.555555558b631p-5);
+    p = __builtin_fma(p, r, 0x1.555555554c5bfp-3);
+    p = __builtin_fma(p, r, 0x1.ffffffffffe94p-2);
+    p = __builtin_fma(p, r, 0x1.0000000000019p+0);
     p = __builtin_fma(p, r, 1.0);
     return __builtin_ldexp(p, n);
 }

@@ -120,3 +120,19 @@ def test_output_in_an_input(dev, orc, shared, T, H, Hkv, n):
     assert np.abs(got.astype(np.float64) - want).max() <= 5e-6 * np.abs(want).max()
     for b in bufs:
         dev.free(b)
+
+
+@pytest.mark.parametrize("T,H,Hkv", [(16384, 64, 4), (16, 32768, 16384)], ids=["tile", "wave"])
+def test_weights_correctly_rounded(dev, T, H, Hkv):
+    """The weights are double exponentials rounded to f32: with scores 0 and -x, x >= 40, and v rows of 0 and 1 a
+    head's output is its second weight, e^-x (1 + e^-x rounds to 1 within 5e-18), which a double good to 2^-51 rounds
+    like the exact value but for one x in 10^8."""
+    x = np.random.default_rng(T).uniform(40.0, 80.0, T * H).astype(np.float32)
+    q = np.zeros((T * H, 4), np.float32)
+    q[:, 0] = -4.0 * x   # 1 / head dim is 1/4
+    k, v = np.zeros((2, Hkv, 4), np.float32), np.zeros((2, Hkv, 4), np.float32)
+    k[1, :, 0] = v[1] = 1.0
+    got = banded(dev, q.reshape(-1), k.reshape(-1), v.reshape(-1), np.zeros(T * H, np.float32), [0] * T, [1] * T,
+                 [1.0] * T, T, H, Hkv, 4, 1, 1, Hkv * 4).reshape(T * H, 4)
+    want = np.exp(-x.astype(np.float64)).astype(np.float32)
+    assert np.array_equal(got, np.broadcast_to(want[:, None], got.shape)), int((got[:, 0] != want).sum())
