@@ -202,7 +202,7 @@ void *sepia_hip_stream(void);
  *                 between routed and shared experts (default 100);
  *   "pf_q" 1/0    prefill projections of layers whose six projections are
  *                 all Q2_K/Q3_K/Q4_K on the int8 matrix cores (1, default),
- *                 or as any other layer (0);
+ *                 or on the bf16 kernels (0);
  *   "pf_h" 1/0    prefill projections of all other layers with 4-byte-aligned
  *                 rows on the f16 matrix cores (1, default), or on the bf16
  *                 kernels (0; they take no Q8_0, so layers that hold it are

@@ -167,12 +167,12 @@ static int g_opt_mq_x = 0;   /* "mq_x": 0 = planner's choice, 1 = vector from gl
 static int g_opt_pf_route_m = 1;   /* "pf_route_m": 1 = prefill router logits on the f32 matrix cores
                                     * (sepia_pf_route_m, _m2) when x and the router rows are 16-byte
                                     * aligned, 0 = sepia_pf_route */
-static int g_opt_pf_h = 1;   /* "pf_h": 1 = prefill layers with 4-byte-aligned rows that the int8 kernels do
-                              * not take run their projections on the f16 matrix cores (sepia_ph_quant,
-                              * sepia_ph_gateup, sepia_ph_down); 0 = on the bf16 kernels */
+static int g_opt_pf_h = 1;   /* "pf_h": 1 = all other prefill layers with 4-byte-aligned rows run their
+                              * projections on the f16 matrix cores (sepia_ph_quant, sepia_ph_gateup,
+                              * sepia_ph_down); 0 = on the bf16 kernels */
 static int g_opt_pf_q = 1;   /* "pf_q": 1 = a prefill layer whose six projections are all Q2_K, Q3_K or Q4_K
                               * runs them on the int8 matrix cores (sepia_pf_quant, sepia_pf_gateup_q,
-                              * sepia_pf_down_q); 0 = as any other layer */
+                              * sepia_pf_down_q); 0 = on the bf16 kernels */
 static int g_opt_tile_t = 0; /* sepia_hip_set_option("tile_t", T) forces T steps per workgroup */
 
 /* Geometry for `mats` stacked copies of a [rows, 256 * n_blocks] matrix; 0
@@ -2210,14 +2210,15 @@ int sepia_gpu_moe_prefill(const SepiaMoeLayerDesc *L, int64_t n_tokens, SepiaGpu
      * rows (its DMA stages Q2_K and Q4_K blocks from their own starts);
      * activations as PQ rows (kernels/prefill_q.h: 832 bytes per 256
      * columns) */
-    const int use_q = g_opt_pf_q && q_aligned && pf_type_int(g.type) && pf_type_int(d.type) &&
-                      (ns == 0 || (pf_type_int(sg.type) && pf_type_int(sd.type)));
+    const int ints = pf_type_int(g.type) && pf_type_int(d.type) &&
+                     (ns == 0 || (pf_type_int(sg.type) && pf_type_int(sd.type)));
+    const int use_q = g_opt_pf_q && q_aligned && ints;
     /* f16 path: layers of the real checkpoint's formats, and mixes of those
      * with the int8 ones (moe_prefill of a Q4_K / Q6_K layer at hidden 4096,
      * 300 tokens: 1.82 ms on the bf16 kernels, 0.59 ms here), rows 4-byte
      * aligned; the bf16 kernels take what is left: layers with rows at 2-byte
      * offsets, and mixes whose activation records pass the bound below */
-    int use_h = !use_q && g_opt_pf_h && q_aligned;
+    int use_h = !ints && g_opt_pf_h && q_aligned;
     if (use_h && !use_h_all && (pf_rows_large(T, H, PF_HREC) || pf_rows_large(P, I, PF_HREC))) use_h = 0;
     /* A capture whose scratch holds the bf16 path's regions, but not the f16
      * path's (up to 2.2 times those), is taken in the fewest even parts of the

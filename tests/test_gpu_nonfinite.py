@@ -14,7 +14,7 @@ import numpy as np
 import pytest
 
 from sepia_amd import hip, synth
-from test_gpu_parity import gpu_matvec_q, make_layer, run_prefill
+from test_gpu_parity import Launches, gpu_matvec_q, make_layer, run_prefill
 
 pytestmark = pytest.mark.gpu
 
@@ -90,21 +90,30 @@ def test_moe_decode_nan_x(dev, orc, types):
         dev.free(b)
 
 
-@pytest.mark.parametrize("kind", ["int8", "f16", "bf16"])
+PREFILL_KERNEL = dict(int8="sepia_pf_gateup_q", f16="sepia_ph_gateup", bf16="sepia_pf_gateup", mixed="sepia_ph_gateup")
+
+
+@pytest.mark.parametrize("kind", list(PREFILL_KERNEL))
 def test_moe_prefill_nonfinite_token(dev, orc, kind):
     """One token of the batch with an infinity: its output row is
     non-finite; every other token's row is bitwise what it is when that
     token is finite (each output element is its own dot product). int8: a
     Q2_K / Q3_K / Q4_K layer on the int8 kernels; f16: a layer of the real
     checkpoint's formats on the f16 kernels; bf16: the Q2_K layer on the bf16
-    kernels."""
+    kernels; mixed: a layer of both kinds on the f16 kernels."""
     rng = np.random.default_rng(12)
-    types = dict(tg=17, tu=17, td=18, ts=13, tsd=14) if kind == "f16" else dict(tg=10, tu=10, td=11, ts=12)
+    types = dict(tg=10, tu=10, td=11, ts=12)
+    if kind == "f16":
+        types = dict(tg=17, tu=17, td=18, ts=13, tsd=14)
+    elif kind == "mixed":
+        types = dict(tg=12, tu=12, td=13, ts=10, tsd=14)
     desc, spec, bufs = make_layer(dev, rng, hidden=2048, inter=1024, n_routed=16, n_shared=2, **types)
     X = rng.standard_normal((24, 2048)).astype(np.float32)
     assert dev.L.sepia_hip_set_option(b"pf_q", 0 if kind == "bf16" else 1) == 1
     try:
-        y0, _, _ = run_prefill(dev, desc, X)
+        with Launches(dev) as n:
+            y0, _, _ = run_prefill(dev, desc, X)
+        assert [k for k in set(PREFILL_KERNEL.values()) if n.count(k)] == [PREFILL_KERNEL[kind]]
         Xb = X.copy()
         Xb[9, 1500] = np.inf
         y1, idx1, _ = run_prefill(dev, desc, Xb)
