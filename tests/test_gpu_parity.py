@@ -934,13 +934,13 @@ PREFILL_CASES = [
     ((2048, 1024, 16, 2), (10, 11, 12), 40),
     ((6144, 3072, 16, 2), (10, 11, 12), 48),      # BASELINE configs[4] shapes, 16 experts resident
     ((2048, 1024, 12, 1), (17, 18, 14), 33),      # IQ2_XS / IQ3_XXS routed, Q6_K shared
-    ((1024, 2048, 8, 2), (13, 23, 11), 20),       # Q5_K / IQ4_XS routed, Q3_K shared (bf16 kernels)
+    ((1024, 2048, 8, 2), (13, 23, 11), 20),       # Q5_K / IQ4_XS routed, Q3_K shared (both families: f16 kernels)
     ((2048, 1024, 12, 1), (11, 10, 10), 37),      # Q3_K / Q2_K routed, Q2_K shared
     # the real checkpoint's format mixes (the f16 kernels on the default path)
     ((6144, 3072, 16, 2), (17, 18, 13, 14), 48),  # IQ2_XS / IQ3_XXS routed, Q5_K / Q6_K shared
     ((2048, 1024, 12, 2), (17, 23, 13, 14), 40),  # IQ4_XS down
     ((1024, 2048, 8, 2), (13, 14, 13, 14), 20),   # Q5_K / Q6_K routed
-    ((256, 512, 8, 1), (17, 18, 13, 14), 11),     # the smallest grids: one 256-row workgroup per slice row
+    ((256, 512, 8, 1), (17, 18, 13, 14), 11),     # rows of 74 bytes: the bf16 kernels on both paths
     ((2048, 1024, 8, 0), (17, 18, 13, 14), 15),   # no shared experts (f16 kernels)
     ((2048, 1024, 8, 0), (10, 11, 12), 15),       # no shared experts (int8 kernels)
     ((2048, 1024, 8, 2), (17, 18, 13, 14), 1),    # one token: every unit a single pair (f16)
@@ -963,12 +963,12 @@ def test_moe_prefill(dev, orc, shape, types, T, x_kind, path):
     """Every token of the batch against the oracle's single-token layer (its
     own routing, near-ties per the reference protocol); two runs bitwise equal.
     x either bf16-representable or full f32. path: a layer of Q2_K / Q3_K /
-    Q4_K projections on the int8 matrix cores, and a layer of the real
-    checkpoint's formats (IQ2_XS, IQ3_XXS, IQ4_XS, Q5_K, Q6_K) on the f16
-    ones (q, the default; options pf_q, pf_h), or either on the bf16 kernels
-    with bit-exact dequantized weights (tile; pf_q 0 and pf_h 0, which also
-    runs the router on sepia_pf_route, pf_route_m 0). Layers with other
-    format mixes take the bf16 kernels on both paths."""
+    Q4_K projections on the int8 matrix cores, and any other layer (IQ2_XS,
+    IQ3_XXS, IQ4_XS, Q5_K, Q6_K, mixes of both kinds) on the f16 ones (q, the
+    default; options pf_q, pf_h), or either on the bf16 kernels with bit-exact
+    dequantized weights (tile; pf_q 0 and pf_h 0, which also runs the router
+    on sepia_pf_route, pf_route_m 0). Layers with rows at 2-byte offsets take
+    the bf16 kernels on both paths."""
     hidden, inter, n_routed, n_shared = shape
     tgu, td, ts = types[:3]
     tsd = types[3] if len(types) > 3 else None
@@ -979,7 +979,14 @@ def test_moe_prefill(dev, orc, shape, types, T, x_kind, path):
     for k, v in PF_PATHS[path].items():
         assert dev.L.sepia_hip_set_option(k.encode(), v) == 1
     try:
-        y, idx, w = run_prefill(dev, desc, X)
+        with Launches(dev) as n:
+            y, idx, w = run_prefill(dev, desc, X)
+        fmts = {tgu, td} | ({ts, ts if tsd is None else tsd} if n_shared else set())
+        aligned = all(synth.row_bytes(t, cols) % 4 == 0 for t, cols in
+                      [(tgu, hidden), (td, inter)] + ([(ts, hidden), (ts if tsd is None else tsd, inter)] if n_shared else []))
+        kernel = "sepia_pf_gateup" if path == "tile" or not aligned else \
+            "sepia_pf_gateup_q" if fmts <= {10, 11, 12} else "sepia_ph_gateup"
+        assert n.count(kernel) == 1, kernel
         y2, _, _ = run_prefill(dev, desc, X)
     finally:
         for k, v in PF_PATHS["q"].items():
