@@ -136,3 +136,9 @@ def test_weights_correctly_rounded(dev, T, H, Hkv):
                  [1.0] * T, T, H, Hkv, 4, 1, 1, Hkv * 4).reshape(T * H, 4)
     want = np.exp(-x.astype(np.float64)).astype(np.float32)
     assert np.array_equal(got, np.broadcast_to(want[:, None], got.shape)), int((got[:, 0] != want).sum())
+
+
+def test_more_tokens_than_a_launch(dev, orc):
+    """Over 32768 tokens, the most a launch takes: the second one starts at its own q, bounds and positions."""
+    T = 32768 + 70
+    check(dev, orc, make(np.random.default_rng(8), T, 1, 1, 4, 8, T, 9))
