@@ -52,8 +52,6 @@
 #define ATT_RP_DCH 64       // d_rel columns staged per pass
 #define ATT_TB 64           // tokens whose bounds travel in the kernel arguments
 #define ATT_BB 256          // tokens per launch of sepia_attn_bounds
-#define ATT_GMAX 16         // query heads per kv head
-#define ATT_DMAX 128        // head dim
 #define ATT_KC 32           // kv rows per step of sepia_attn_tile
 #define ATT_KS 136          // floats of a staged k row (34 16-byte pieces, 2 mod 4: no bank conflicts)
 #define ATT_VS 144          // floats of a staged v row (rows 4 apart differ by 16 banks)

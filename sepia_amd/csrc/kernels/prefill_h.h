@@ -451,7 +451,7 @@ template <bool B> struct PhBool { static constexpr bool value = B; };
 // One projection workgroup (see the top of the file). GU: wave w computes
 // rows r0 + 16 w .. of gate (W0, tile 0) and up (W1, tile 1), h[pair][row] =
 // silu(gate) * up in f32; down: rows r0 + 32 w .. of W0, out[pair][row] in
-// f32. rows: those of the matrix; a wave past them only stages records.
+// f32. rows: those of the matrix, a multiple of 256 as the host checks.
 template <int T, bool GU, int MT>
 __device__ __forceinline__ void ph_proj(uint8_t *smem, const uint8_t *W0, const uint8_t *W1, uint64_t row_bytes,
                                         int64_t nb, const uint8_t *rec, const int64_t *roff, const int32_t *pair,
@@ -468,7 +468,11 @@ __device__ __forceinline__ void ph_proj(uint8_t *smem, const uint8_t *W0, const 
     const int tid = (int)threadIdx.x, l = tid & 63, n = l & 15, g = l >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t grow = r0 + 16 * HT * w;   // the wave's first row
-    const bool on = grow < rows;
+    // Always true, which the compiler does not know: a branch on it ends the
+    // basic block at every half of the unrolled loop below. As straight-line
+    // code the kernels spilled 889 registers (9 tokens 539 -> 556 us, 300
+    // tokens of a mixed layer 557 -> 592).
+    const bool whole = grow < rows;
     const int nbi = (int)nb, nst = 2 * nbi;
     const uint8_t *tab = smem + PH_O_TAB, *signs = smem + PH_O_SIGNS;
     ph_fill_tables<T>(smem);   // published by the first barrier
@@ -504,7 +508,7 @@ __device__ __forceinline__ void ph_proj(uint8_t *smem, const uint8_t *W0, const 
     };
     // weights: piece q = 64 k + lane of a tile's group is row q / PW, bytes
     // 16 (q % PW) .. of it; pieces past the row's last block take the group's
-    // first (the last one that holds block bytes may run up to 14 bytes past
+    // first (the last one that holds block bytes may run up to 12 bytes past
     // the matrix, into the 256 that every device buffer of the library
     // carries past its data, dev_bytes in sepia_hip.c)
     uint32_t wrow[KW], wcol[KW];
@@ -515,8 +519,8 @@ __device__ __forceinline__ void ph_proj(uint8_t *smem, const uint8_t *W0, const 
         wcol[k] = 16u * (uint32_t)(q - m * PW);
     }
     // (from the wave's first row: 32-bit offsets then reach its rows in a matrix of any size)
-    const uint64_t wfirst = on ? (uint64_t)grow * row_bytes : 0;
-    const uint8_t *Wt[NT] = {W0 + wfirst, GU ? W1 + wfirst : W0 + wfirst + (on ? 16 * row_bytes : 0)};
+    const uint64_t wfirst = (uint64_t)grow * row_bytes;
+    const uint8_t *Wt[NT] = {W0 + wfirst, GU ? W1 + wfirst : W0 + wfirst + 16 * row_bytes};
     uint8_t *wl = smem + O_W + (uint32_t)w * (NT * 16 * 16 * PW);
     ph_u4 wr[NT][KW];
     auto w_load = [&](int b) {   // the group of blocks b ..
@@ -657,9 +661,8 @@ __device__ __forceinline__ void ph_proj(uint8_t *smem, const uint8_t *W0, const 
             }
         }
     };
-    // Every load is unconditional (past the last block, the last one again;
-    // waves without rows, row 0): a wait after a branch around loads would be
-    // for all of them.
+    // Every load is unconditional (past the last block, the last one again): a
+    // wait after a branch around loads would be for all of them.
 #pragma unroll
     for (int i = 0; i < AD; i++) a_load(i, i);
     w_load(0);
@@ -680,8 +683,8 @@ __device__ __forceinline__ void ph_proj(uint8_t *smem, const uint8_t *W0, const 
                 w_load(b + G < nbi ? b + G : b);
                 asm volatile("" ::: "memory");
             }
-            if (on) {
-                const int o = (i / 2 % G) * F::BB + (G == 1 && F::BB % 4 ? i / 2 * 2 : 0);
+            const int o = (i / 2 % G) * F::BB + (G == 1 && F::BB % 4 ? i / 2 * 2 : 0);
+            if (whole) {
                 if (F::BB % 4 && (i / 2) % 2) half(PhBool<true>{}, o, hb);
                 else half(PhBool<false>{}, o, hb);
             }
@@ -695,7 +698,6 @@ __device__ __forceinline__ void ph_proj(uint8_t *smem, const uint8_t *W0, const 
             __syncthreads();
         }
     }
-    if (!on) return;
     // y = s_pair * acc; lane: pairs 16 mt + 4 g + k, rows grow + 16 t + n
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
