@@ -79,11 +79,6 @@
 #pragma once
 #include "prefill_q.h"
 
-// The two unrolled kernels, half a megabyte of code each, stand after all
-// others in the code object, so that the decode kernels stay within its first
-// 2 MB: behind them, with the same machine code, four MoE decode layers took
-// 259-264 us against 255-256, and 258 against 257 so.
-#define PH_LAST __attribute__((section(".text.ph")))
 #define PH_UM 64                       // pairs per unit
 #define PH_REC 576                     // bytes of a 128-column PH record
 #define PH_LREC 608                    // a staged record (38 16-byte pieces, 2 mod 4: no LDS bank conflicts)
@@ -770,7 +765,7 @@ __device__ __forceinline__ int64_t ph_nb(int32_t t, int64_t n_blocks) { return t
 // The host launches it only when every projection of the layer has one of
 // the formats above, with 4-byte-aligned rows, and H and I are multiples of
 // 256.
-extern "C" __global__ PH_LAST __launch_bounds__(64 * PH_WAVES) void sepia_ph_gateup(
+extern "C" __global__ __launch_bounds__(64 * PH_WAVES) void sepia_ph_gateup(
     PfProj gate, PfProj up, PfProj s_gate, PfProj s_up, int32_t n_routed, int32_t n_sel, int64_t I, int64_t H,
     const uint8_t *__restrict__ phx, const float *__restrict__ phxs, const int32_t *__restrict__ list,
     const int32_t *__restrict__ units, const int32_t *__restrict__ n_units, float *__restrict__ hf) {
@@ -792,7 +787,7 @@ extern "C" __global__ PH_LAST __launch_bounds__(64 * PH_WAVES) void sepia_ph_gat
 
 // Down: workgroup (256-row slice bx of H, unit by); yp[p][row] = down_e .
 // h_p in f32 (h_p the PH row p). Same launch conditions.
-extern "C" __global__ PH_LAST __launch_bounds__(64 * PH_WAVES) void sepia_ph_down(
+extern "C" __global__ __launch_bounds__(64 * PH_WAVES) void sepia_ph_down(
     PfProj down, PfProj s_down, int32_t n_routed, int64_t I, int64_t H, const uint8_t *__restrict__ phh,
     const float *__restrict__ phhs, const int32_t *__restrict__ list, const int32_t *__restrict__ units,
     const int32_t *__restrict__ n_units, float *__restrict__ yp) {
