@@ -125,7 +125,8 @@ int sepia_hip_set_iq2xxs_grid(const uint64_t *grid256);
  * rows) to at least `bytes` now, so that later calls of the same or smaller
  * shapes allocate nothing. A call whose scratch would have to grow while the
  * stream is being captured fails instead (an allocation cannot be captured):
- * run the call once, or reserve, before beginning a capture. Needs init. */
+ * run the call once, or reserve, before beginning a capture. (banded_attn
+ * takes fewer splits first, moe_prefill may run in parts, above.) Needs init. */
 int sepia_hip_reserve_scratch(size_t bytes);
 
 /* Bytes of the library's growable scratch region (0 before its first use).

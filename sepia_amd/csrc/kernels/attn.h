@@ -40,7 +40,7 @@
 // Measured (64 heads of 128): one token over 20001 kv rows of 8 heads (164
 // MB of k and v) 41.9 + 7.8 us, 3.9 TB/s, against 279 + 47 us for scalar
 // loops that reduced each score over 16 lanes by shuffles; 500 tokens over
-// 1500 + 500 rows 547 us, 105 TFLOP/s over both products, against 6.1 ms.
+// 1500 + 500 rows 548 us, 105 TFLOP/s over both products, against 6.1 ms.
 // Both kernels need two waves a SIMD: with 400 registers and one wave they
 // took 68 and 877 us, with spills 98 and 605 us. At 4 tokens over 6004 rows
 // (8 heads a kv head: 32 rows) the wave kernel takes 27.8 us, at 8 tokens the

@@ -18,8 +18,12 @@
 //                     Q4_K runs them on the int8 matrix cores (prefill_q.h:
 //                     sepia_pf_quant, sepia_pf_gateup_q, sepia_pf_down_q); any
 //                     other layer on the f16 ones (prefill_h.h:
-//                     sepia_ph_quant, sepia_ph_gateup, sepia_ph_down); layers
-//                     with rows at 2-byte offsets on the bf16 ones here:
+//                     sepia_ph_quant, sepia_ph_gateup, sepia_ph_down); both
+//                     need rows at 4-byte offsets. The rest on the bf16 ones
+//                     here: rows at 2-byte offsets, mixes of both format
+//                     families in batches past pf_rows_large (sepia_hip.c) or
+//                     captured with scratch that not even one token's part
+//                     fits on the f16 ones, and options pf_q, pf_h:
 //     sepia_pf_split    x as bf16 hi / lo
 //     sepia_pf_gateup   per (32-row tile, unit): h[p][.] = silu(g) * u (bf16 hi / lo)
 //     sepia_pf_down     per (64-row tile, unit): yp[p][.] = down_e . h[p]
